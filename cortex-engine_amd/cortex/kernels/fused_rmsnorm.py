@@ -5,7 +5,7 @@ Drop-in for ``cortex.kernels.fused_rmsnorm`` of the reference
 signature (``w`` pre-transposed ``(K, N)``) and semantics
 ``((x_f32 / rms) * gamma).to(x.dtype) @ w (+ bias)``: per-row statistics in fp32,
 the normalised row rounded to x's dtype while it is staged into LDS, the contraction
-on MFMA (bf16 for bf16 inputs, fp32 for fp32 inputs) with fp32 accumulation.
+on MFMA with fp32 accumulation (fp32 inputs as exact sums of bf16 parts).
 ``norm_linear_int8`` is the same kernel on QuantizedLinear's int8 ``(N, K)``
 weights with the per-channel scale applied in the epilogue.
 """
@@ -59,7 +59,7 @@ def norm_linear_int8(x: torch.Tensor, weight_int8: torch.Tensor, weight_scale: t
 
     ``weight_int8`` is ``(N, K)`` int8 and ``weight_scale`` ``(N,)`` fp32 as stored by
     QuantizedLinear (reference calibrate.py:192-193).  bf16 inputs use bf16 MFMA,
-    fp32 inputs fp32 MFMA; the int8 weights are widened exactly.
+    fp32 inputs their exact bf16 parts; the int8 weights are widened exactly.
     """
     nat.require_gpu(x, weight_int8, weight_scale, gamma, beta, bias, residual, what="norm_linear_int8")
     compute = torch.bfloat16 if x.dtype == torch.bfloat16 else torch.float32

@@ -588,6 +588,8 @@ def convert(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
 # normalises the rows (bit-for-bit the model's CORTEX_INT8_WEIGHTS switch, same variable)
 INT8_WEIGHTS = os.environ.get("CORTEX_INT8_WEIGHTS", "image")
 
+SPLIT_MIN_N = 8  # outputs up to this wide without a norm stay one dot product per row (fp32 compute)
+
 _KN_CACHE: "OrderedDict[tuple, tuple]" = OrderedDict()
 _KN_CACHE_SIZE = 16
 # keys whose rows a captured HIP graph reads: never evicted (the graph holds their address)
@@ -776,13 +778,30 @@ def norm_linear(x: torch.Tensor, *, weight: torch.Tensor | None = None, weight_i
             kw = {"weight": w2, "weight_scale": ws}
         return norm_linear(xn, **kw, bias=bias, act=act, residual=residual, res_rows=res_rows,
                            out_dtype=out_dtype, compute_dtype=compute_dtype, out=out)
-    if nrm and stats is None:
-        stats = row_stats(x2, "layer" if nrm == 1 else "rms", eps)
     res2 = None
     if residual is not None:
         res2 = residual.reshape(-1, N) if residual.dim() != 2 else residual
         res2 = _row_major_2d(res2)
     ld_w = w2.stride(0) if w2.shape[0] > 1 else w2.shape[1]
+    if (compute_dtype == torch.float32 and x2.dtype == out2.dtype == torch.float32 and stats is None
+            and w2.dtype in (torch.float32, torch.int8) and (nrm or N > SPLIT_MIN_N) and M > 0
+            and all(t is None or t.dtype == torch.float32 for t in (ws, bias, res2))
+            and (not nrm or (gamma is not None and gamma.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                             and (beta is None or beta.dtype == gamma.dtype)
+                             and all(t is None or t.is_contiguous() for t in (gamma, beta))))):
+        # fp32 on the bf16 matrix cores: operands as exact sums of bf16 parts (gemm_split.hip)
+        ws_bytes = nat.load().cortex_norm_linear_split_workspace_bytes(M, N, K, nat.code(w2.dtype))
+        if ws_bytes > 0:
+            ws_t = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            nat.call("cortex_norm_linear_split", M, N, K, nat.ptr(x2), x2.stride(0) if M > 1 else K, nrm,
+                     nat.ptr(gamma), nat.ptr(beta), nat.code(gamma.dtype) if nrm else nat.F32, float(eps),
+                     nat.code(w2.dtype), layout, nat.ptr(w2), ld_w, nat.ptr(ws), nat.ptr(bias), ACT[act],
+                     nat.ptr(res2), (res2.stride(0) if res2.shape[0] > 1 else N) if res2 is not None else 0,
+                     int(res_rows), nat.ptr(out2), out2.stride(0) if M > 1 else N, nat.ptr(ws_t), ws_bytes,
+                     nat.stream_of(dev))
+            return out
+    if nrm and stats is None:
+        stats = row_stats(x2, "layer" if nrm == 1 else "rms", eps)
     if (res2 is not None and not nrm and not ACT[act] and layout == 0 and weight is not None
             and w2.dtype == torch.bfloat16 and x2.dtype == torch.bfloat16 and res2.dtype == torch.float32
             and out2.dtype == torch.float32 and (bias is None or bias.dtype == torch.float32)

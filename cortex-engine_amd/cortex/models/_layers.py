@@ -21,7 +21,8 @@ bf16 compute (the default):
     image speed and no launch is added (``WeightWindow``).
     For a float nn.Linear the image is the weight rounded to bf16, as ``F.linear`` on
     bf16 inputs would use it.
-fp32 compute: int8 or fp32 weights, fp32 operands, fused norm prologue.
+fp32 compute: int8 or fp32 weights, fp32 operands as exact sums of bf16 parts (gemm_split.hip), the
+norm applied where the rows are split.
 """
 
 from __future__ import annotations

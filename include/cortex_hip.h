@@ -253,6 +253,23 @@ int cortex_norm_linear(int64_t M, int64_t N, int64_t K, int x_dtype, const void*
                        int64_t ld_res, int64_t res_rows, int out_dtype, void* out, int64_t ld_out,
                        hipStream_t stream);
 
+/* The fp32-compute form of cortex_norm_linear on the bf16 matrix cores (the fp32 rows of
+ * cortex/kernels/fused_rmsnorm.py:239-301 and of QuantizedLinear, calibrate.py:225-228): every
+ * fp32 operand as the exact sum of three bf16 parts, products and sums in fp32 (an int8 weight is
+ * one part).  x, residual and out fp32; w int8 (N, K) or fp32 in (N, K) (w_layout 0) or (K, N) (1);
+ * norm 0 none, 1 LayerNorm, 2 RMS, its statistics computed by the call (gamma and beta in
+ * gamma_dtype 0, 1 or 2); w_scale, bias optional fp32; act, residual and res_rows as
+ * cortex_norm_linear; out may be residual.  The workspace (16-byte aligned) holds the parts of the
+ * weight and of as many rows as fit: cortex_norm_linear_split_workspace_bytes gives the size that
+ * takes up to 256 MiB of rows at once (0: a weight too large for this form); a smaller one, down to
+ * 128 rows, only costs more launches. */
+int64_t cortex_norm_linear_split_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
+int cortex_norm_linear_split(int64_t M, int64_t N, int64_t K, const float* x, int64_t ld_x, int norm,
+                             const void* gamma, const void* beta, int gamma_dtype, float eps, int w_dtype,
+                             int w_layout, const void* w, int64_t ld_w, const float* w_scale, const float* bias,
+                             int act, const float* residual, int64_t ld_res, int64_t res_rows, float* out,
+                             int64_t ld_out, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
 /* Norm + linear in ONE launch (rms_norm_linear, cortex/kernels/fused_rmsnorm.py:130-233 and
  * :239-301, with QuantizedLinear's int8 weights, calibrate.py:170-235):
  *   y[m, :]  = bf16( x[m, :] / sqrt(mean_k x[m, k]^2 + eps) * gamma )             (norm 2, RMS)
