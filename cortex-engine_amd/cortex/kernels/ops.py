@@ -858,8 +858,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float
     s = float(scale) if scale is not None else Dh ** -0.5
     km_sb = 0
     if key_mask is not None:
-        key_mask = key_mask.to(torch.uint8) if key_mask.dtype == torch.bool else key_mask
         key_mask = key_mask.contiguous()
+        if key_mask.dtype == torch.bool:
+            key_mask = key_mask.view(torch.uint8)
         km_sb = key_mask.stride(0) if key_mask.dim() == 2 else 0
     bm_sb = n_qt = n_kt = 0
     if block_mask is not None:

@@ -52,14 +52,19 @@ class CrossAttentionBlock(nn.Module):
         B, L, D = latents.shape
         E = tokens.shape[1]
         H = self.num_heads
-        q = apply_linear(self.q_proj, latents, norm=self.norm_q, out_dtype=compute, compute=compute)
+        # latents expanded over the batch (the encoder's call): their L rows once, read by every sample
+        shared = B > 1 and latents.stride(0) == 0 and not self.q_proj._forward_pre_hooks
+        lat = latents[:1] if shared else latents
+        n = lat.shape[0]
+        q = apply_linear(self.q_proj, lat, norm=self.norm_q, out_dtype=compute, compute=compute)
         kv = apply_linear(self.kv_proj, tokens, norm=self.norm_kv, out_dtype=compute, compute=compute)
-        q2, kv2 = q.reshape(B * L, D), kv.reshape(B * E, 2 * D)
+        q2, kv2 = q.reshape(n * L, D), kv.reshape(B * E, 2 * D)
         o_buf, o = ops.merge_heads_out(B, L, H, D // H, compute, latents.device)
-        ops.attention(ops.heads_view(q2, B, L, H), ops.heads_view(kv2, B, E, H, 0, D),
-                      ops.heads_view(kv2, B, E, H, D, D), key_mask=token_mask, out=o)
-        return apply_linear(self.out_proj, o_buf, residual=latents.reshape(B * L, D).contiguous(),
-                            out_dtype=latents.dtype, compute=compute).reshape(B, L, D)
+        ops.attention(ops.heads_view(q2, n, L, H), ops.heads_view(kv2, B, E, H, 0, D),
+                      ops.heads_view(kv2, B, E, H, D, D), key_mask=token_mask, out=o, batch=B)
+        return apply_linear(self.out_proj, o_buf, residual=lat.reshape(n * L, D).contiguous(),
+                            res_rows=L if shared else 0, out_dtype=latents.dtype,
+                            compute=compute).reshape(B, L, D)
 
 
 class SelfAttentionBlock(nn.Module):

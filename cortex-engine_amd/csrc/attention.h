@@ -25,7 +25,7 @@ struct AttnArgs {
   int vec;
 };
 
-// bf16, head dim 64, no per-key or block mask, 16-byte aligned rows
+// bf16, head dim 64, a per-key or a tile mask or none, 16-byte aligned rows
 // (attention_fast.hip).  Returns 1 when it launched, 0 when the request is outside
 // its specialisation (the caller then runs the general kernel), negative on error.
 int try_attention_fast(const AttnArgs& a, int dtype, hipStream_t stream);

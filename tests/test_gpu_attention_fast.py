@@ -104,6 +104,37 @@ def test_fast_and_general_kernels_agree():
     assert err <= 1e-2 * float(general.abs().max())
 
 
+@pytest.mark.parametrize("E", [1, 63, 64, 65, 320, 777, 4200])
+@pytest.mark.parametrize("B,L,shared", [(3, 200, False), (40, 256, True)])
+def test_key_mask_bf16(E, B, L, shared):
+    """Per-key masks in the fast kernel: a prefix, holes over whole tiles, single keys, none, all; one
+    mask per sample or one for all; the rows of a masked key may hold anything finite."""
+    from cortex.kernels import ops
+
+    g = torch.Generator().manual_seed(E + B)
+    q, k, v = ((torch.randn(B, H, n, DH, generator=g) / 2).bfloat16() for n in (L, E, E))
+    m = torch.rand(B, E, generator=g) < 0.6
+    m[0] = torch.arange(E) < (E + 1) // 2
+    m[1, : E // 2] = False
+    m[2] = False
+    m[-1] = E > 64
+    m[-1, E // 3] = True
+    k[:, :, :][~m[:, None, :, None].expand_as(k)] = 100.0
+    if shared:
+        m = m[1]
+        if not m.any():
+            m[-1] = True
+    kpm = m.to(DEV)
+    got = ops.attention(q.to(DEV), k.to(DEV), v.to(DEV), key_mask=kpm).float().cpu().numpy()
+    for b in sorted({0, 1, 2, B - 1}):
+        mb = m if shared else m[b]
+        if not mb.any():
+            assert (got[b] == 0).all()
+            continue
+        ref = O.attention_bruteforce_f64(q[b:b + 1].float(), k[b:b + 1][:, :, mb].float(), v[b:b + 1][:, :, mb].float())
+        _close(got[b:b + 1], ref)
+
+
 @pytest.mark.parametrize("B,L,D", [(3, 256, 512), (2, 200, 512), (4, 64, 256), (2, 1, 512), (33, 256, 512)])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_fused_qkv_attention(B, L, D, with_bias):
