@@ -30,4 +30,8 @@ struct AttnArgs {
 // its specialisation (the caller then runs the general kernel), negative on error.
 int try_attention_fast(const AttnArgs& a, int dtype, hipStream_t stream);
 
+// fp32, head dim 64, any masks with 64-key granularity, 16-byte aligned rows (attention_split.hip);
+// same return values.
+int try_attention_split(const AttnArgs& a, int dtype, hipStream_t stream);
+
 }  // namespace cortex

@@ -336,7 +336,8 @@ extern "C" int cortex_attention(int dtype, int64_t B, int64_t H, int64_t Lq, int
   for (const void* p : {q, k, v}) vec = vec && ((uintptr_t)p % 16 == 0);
   for (int64_t s : {q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl}) vec = vec && ((s * es) % 16 == 0);
   a.vec = vec ? 1 : 0;
-  const int fast = try_attention_fast(a, dtype, stream);
+  int fast = try_attention_fast(a, dtype, stream);
+  if (fast == 0) fast = try_attention_split(a, dtype, stream);
   if (fast != 0) return fast > 0 ? OK : fast;
   if (dtype == DT_BF16) return launch_attn<bf16>(a, stream);
   if (dtype == DT_F32) return launch_attn<float>(a, stream);
