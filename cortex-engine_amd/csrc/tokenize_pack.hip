@@ -3,7 +3,7 @@
 //   * pack plan: a device-side stable counting sort of the events by batch index
 //     (no host synchronisation): per-chunk histograms, one scan over (chunk,
 //     sample), then in-order ranking inside each chunk -- one launch for small
-//     plans, three for large ones.
+//     plans, two for larger ones (three past 1024 samples).
 //     It yields CSR offsets (B+1), the CSR row of every event and the source
 //     event of every CSR row -- exactly the stable argsort + exclusive cumsum of
 //     the reference pack (cortex/models/cortex.py:140-160).
@@ -78,8 +78,8 @@ __global__ void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
   if (i < n) p[i] = v;
 }
 
-// Whether every range of the wide sorted check (pack_sorted_kernel's status words: 1 sorted
-// and in range, 2 not) was sorted; the whole workgroup takes part and gets the same answer.
+// Whether every chunk of the sorted check (pack_count_kernel's status words: 1 sorted and in
+// range, 2 not) was sorted; the whole workgroup takes part and gets the same answer.
 // A null status list means no check ran.
 __device__ bool ranges_sorted(const int* __restrict__ status, int n_status, int* s_flag) {
   if (!status) return false;
@@ -90,143 +90,6 @@ __device__ bool ranges_sorted(const int* __restrict__ status, int n_status, int*
   __syncthreads();
   return *s_flag != 0;
 }
-
-// The three launches below return at once when the wide sorted check found every range
-// sorted (the identity plan it wrote is the plan).
-
-// 1) per-chunk histogram of batch indices.
-__global__ __launch_bounds__(256) void pack_count_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx, int64_t E,
-                                                          int B, int64_t C, int* __restrict__ counts,
-                                                          int* __restrict__ err, const int* __restrict__ status,
-                                                          int n_status) {
-  __shared__ int hist[PACK_MAX_B];
-  __shared__ int sorted_flag;
-  if (ranges_sorted(status, n_status, &sorted_flag)) return;
-  const int chunk = blockIdx.x;
-  for (int b = threadIdx.x; b < B; b += blockDim.x) hist[b] = 0;
-  __syncthreads();
-  const int64_t beg = (int64_t)chunk * C;
-  const int64_t end = min(E, beg + C);
-  bool bad = false;
-  const int lane = threadIdx.x & 63, bits = sample_bits(B);
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int64_t i0 = beg; i0 < end; i0 += blockDim.x) {  // every lane runs the same trip count
-    const int64_t i = i0 + threadIdx.x;
-    int64_t b = -1;
-    if (i < end) {
-      b = bidx[i * s_bidx];
-      if (b < 0 || b >= B) {
-        bad = true;
-        b = -1;
-      }
-    }
-    // one atomic per distinct sample among the wave's 64 events, by its lowest lane
-    // (sorted batches would otherwise send 64 atomics to one LDS word)
-    const uint64_t same = same_sample_lanes((int)b, b >= 0, bits);
-    if (b >= 0 && (same & lt_mask) == 0) atomicAdd(&hist[b], (int)__popcll(same));
-  }
-  if (bad && err) atomicOr(err, ERR_BATCH_INDEX);
-  __syncthreads();
-  for (int b = threadIdx.x; b < B; b += blockDim.x) counts[(int64_t)chunk * B + b] = hist[b];
-}
-
-// 2) exclusive scan over chunks per sample (in place), then over samples.
-__global__ __launch_bounds__(1024) void pack_scan_kernel(int* __restrict__ counts, int nchunks, int B,
-                                                          int64_t* __restrict__ offsets, int32_t* __restrict__ ident,
-                                                          const int* __restrict__ status, int n_status) {
-  __shared__ int64_t part[1024];
-  __shared__ int totals[PACK_MAX_B];
-  __shared__ int sorted_flag;
-  const int tid = threadIdx.x;
-  if (ranges_sorted(status, n_status, &sorted_flag)) {
-    if (ident && tid == 0) *ident = 1;
-    return;
-  }
-  for (int b = tid; b < B; b += blockDim.x) {
-    int run = 0;
-    for (int c = 0; c < nchunks; ++c) {
-      int t = counts[(int64_t)c * B + b];
-      counts[(int64_t)c * B + b] = run;
-      run += t;
-    }
-    totals[b] = run;
-  }
-  __syncthreads();
-  // each thread owns a contiguous span of samples
-  const int per = (B + blockDim.x - 1) / blockDim.x;
-  const int b0 = tid * per;
-  int64_t local = 0;
-  for (int b = b0; b < min(B, b0 + per); ++b) local += totals[b];
-  part[tid] = local;
-  __syncthreads();
-  // Hillis-Steele inclusive scan of the 1024 partials
-  for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-    int64_t v = (tid >= off) ? part[tid - off] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  int64_t run = part[tid] - local;  // exclusive prefix of this span
-  for (int b = b0; b < min(B, b0 + per); ++b) {
-    offsets[b] = run;
-    run += totals[b];
-  }
-  if (tid == blockDim.x - 1) offsets[B] = part[tid];
-  if (ident && tid == 0) *ident = 0;  // this plan always writes `order`
-}
-
-// 3) in-order ranking inside each chunk: one wavefront walks its chunk 64 events
-//    at a time; lanes holding the same sample are ranked by lane order.
-__global__ __launch_bounds__(64) void pack_rank_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx, int64_t E,
-                                                        int B, int64_t C, const int* __restrict__ chunk_base,
-                                                        const int64_t* __restrict__ offsets,
-                                                        int64_t* __restrict__ order, int64_t* __restrict__ dst_rows,
-                                                        int64_t* __restrict__ rank, const int* __restrict__ status,
-                                                        int n_status) {
-  __shared__ int64_t next[PACK_MAX_B];
-  __shared__ int sorted_flag;
-  if (ranges_sorted(status, n_status, &sorted_flag)) return;
-  const int chunk = blockIdx.x;
-  const int lane = threadIdx.x;
-  for (int b = lane; b < B; b += 64) next[b] = offsets[b] + chunk_base[(int64_t)chunk * B + b];
-  __syncthreads();
-  const int64_t beg = (int64_t)chunk * C;
-  const int64_t end = min(E, beg + C);
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int bits = sample_bits(B);
-  for (int64_t base = beg; base < end; base += 64) {
-    const int64_t i = base + lane;
-    int64_t b = -1;
-    if (i < end) {
-      b = bidx[i * s_bidx];
-      if (b < 0 || b >= B) b = -1;  // counted as an error by pack_count_kernel
-    }
-    const uint64_t same = same_sample_lanes((int)b, b >= 0, bits);
-    int64_t row0 = 0;
-    if (b >= 0) {
-      row0 = next[b];  // every lane of a sample reads the same word ...
-      const int64_t row = row0 + __popcll(same & lt_mask);
-      order[row] = i;
-      if (dst_rows) dst_rows[i] = row;
-      if (rank) rank[i] = row - offsets[b];
-    }
-    __syncthreads();  // single wavefront: the reads above complete before the update
-    if (b >= 0 && (same & lt_mask) == 0) next[b] = row0 + __popcll(same);  // ... and its lowest lane advances it
-    __syncthreads();
-  }
-}
-
-// Small plans (B <= 1024, E <= 65536) in ONE launch: one workgroup of 16 waves, wave w
-// owning the contiguous event chunk w.  Per-wave histograms in LDS, the two scans
-// (over waves per sample, then over samples), then the same in-order ranking as
-// pack_rank_kernel.  Same results as the three-launch path, a third of its launches.
-// Without ranks, sorted indices are recognised first and take the identity plan.  When the
-// caller asks for an identity flag, a sorted plan sets it and leaves `order` unwritten (a
-// consumer then maps row r to event r); an unsorted one clears it and writes `order`.
-constexpr int PS_WAVES = 16;
-constexpr int PS_MAX_B = 1024;
-constexpr int64_t PS_MAX_E = 65536;
-constexpr int PS_UNROLL = 16;
 
 // Sorted batch indices (the collate order) need no sort: the plan is the identity and
 // offsets[s] is the first event of sample s.  Event e (index b, the event before it bp; -1
@@ -257,47 +120,344 @@ __device__ __forceinline__ int64_t prev_index(int64_t b, int64_t e, int64_t E, c
   return (e > 0 && e < E) ? bidx[(e - 1) * s_bidx] : -1;
 }
 
-// Above PS_ONE_E events the sorted check runs wide first: one workgroup per PS_SORTED_EV
-// events (one per thread) applies sorted_event to its range and records in
-// status[blockIdx.x] whether the range (with the event before it) was sorted and in range: 1
-// yes, 2 no.  pack_small_kernel then returns at once when every status is 1 and otherwise
-// recomputes the whole plan.  Up to PS_ONE_E events pack_small_kernel makes the check itself
-// (one round of loads per thread), so a plan is one launch; above that one workgroup is
-// latency-bound (9.5 us at 16384 events against about 2 + 1.5 us for the wide check and the
-// status read).
-constexpr int PS_SORTED_EV = 256;
-constexpr int PS_ONE_UNROLL = 4;
-constexpr int64_t PS_ONE_E = 64 * PS_WAVES * PS_ONE_UNROLL;
-
-__global__ __launch_bounds__(PS_SORTED_EV) void pack_sorted_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx,
-                                                                   int64_t E, int B, int64_t* __restrict__ offsets,
-                                                                   int64_t* __restrict__ order,
-                                                                   int64_t* __restrict__ dst_rows,
-                                                                   int* __restrict__ status, int32_t* clear_err,
-                                                                   WidenRider wr) {
+// The launches after this one return at once when the check below found every range sorted (the identity
+// plan it wrote is the plan).
+//
+// 1) per-chunk histogram of batch indices and, with `status`, the check for sorted indices: a chunk
+// whose events (with the event before it) are in order and in range writes its part of the identity
+// plan and status 1, another one nothing and status 2.  (Only whole sorted chunks write: of shuffled
+// events every second one would otherwise fill the offsets between two samples, 38 us for 84992 events
+// in 256 samples, 3 without.)  Bound by latency: four loads in flight per thread, one LDS pass.
+// The error word is only cleared here, never set: the next launch sets it.
+constexpr int PC_UNROLL = 4;  // events per thread and round (a round: 1024 events, the usual chunk)
+__global__ __launch_bounds__(256) void pack_count_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx, int64_t E,
+                                                          int B, int64_t C, int* __restrict__ counts,
+                                                          int64_t* __restrict__ offsets, int64_t* __restrict__ order,
+                                                          int64_t* __restrict__ dst_rows, int* __restrict__ status,
+                                                          int32_t* clear_err, WidenRider wr) {
   // the plan's workgroups first; a widening rider's after them, on the CUs the plan leaves idle
   const int nplan = (int)gridDim.x - wr.blocks;
   if ((int)blockIdx.x >= nplan) {
     widen_rider_run(wr, (int)blockIdx.x - nplan);
     return;
   }
-  __shared__ int bad;
-  if (threadIdx.x == 0) bad = 0;
-  if (clear_err && blockIdx.x == 0 && threadIdx.x == 0) clear_err_word(clear_err, &bad);
+  __shared__ int hist[PACK_MAX_B];
+  __shared__ int sink;
+  const int chunk = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  if (clear_err && chunk == 0 && tid == 0) clear_err_word(clear_err, &sink);
+  const int64_t beg = (int64_t)chunk * C, end = min(E, beg + C);
+  int64_t bv[PC_UNROLL], bp[PC_UNROLL];
+  auto load = [&](int64_t i0) {
+#pragma unroll
+    for (int u = 0; u < PC_UNROLL; ++u) {
+      const int64_t e = i0 + u * 256 + tid;
+      bv[u] = e < end ? bidx[e * s_bidx] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < PC_UNROLL; ++u) bp[u] = prev_index(bv[u], i0 + u * 256 + tid, end, bidx, s_bidx, lane);
+  };
+  load(beg);
+  for (int b = tid; b < B; b += 256) hist[b] = 0;
   __syncthreads();
-  const int64_t e = (int64_t)blockIdx.x * PS_SORTED_EV + threadIdx.x;
-  const int64_t b = e < E ? bidx[e * s_bidx] : 0;
-  const int64_t bp = prev_index(b, e, E, bidx, s_bidx, threadIdx.x & 63);
-  if (e < E && !sorted_event(e, b, bp, E, B, offsets, order, dst_rows)) bad = 1;
-  __syncthreads();
-  if (threadIdx.x == 0) status[blockIdx.x] = bad ? 2 : 1;
+  const int bits = sample_bits(B);
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int bad = 0;
+  for (int64_t i0 = beg; i0 < end; i0 += PC_UNROLL * 256) {
+    if (i0 > beg) load(i0);
+#pragma unroll
+    for (int u = 0; u < PC_UNROLL; ++u) {
+      const int64_t e = i0 + u * 256 + tid, b = bv[u];
+      const bool valid = b >= 0 && b < B;
+      if (e < end && (!valid || bp[u] > b || (e > 0 && bp[u] < 0))) bad = 1;
+      // one atomic per distinct sample among the wave's 64 events, by its lowest lane
+      // (sorted batches would otherwise send 64 atomics to one LDS word)
+      const uint64_t same = same_sample_lanes((int)b, valid, bits);
+      if (valid && (same & lt_mask) == 0) atomicAdd(&hist[b], (int)__popcll(same));
+    }
+  }
+  bad = __syncthreads_or(bad);  // (the histogram is complete too)
+  for (int b = tid; b < B; b += 256) counts[(int64_t)chunk * B + b] = hist[b];
+  if (!status) return;
+  if (tid == 0) status[chunk] = bad ? 2 : 1;
+  if (bad) return;
+  for (int64_t i0 = beg; i0 < end; i0 += PC_UNROLL * 256) {
+    if (C > PC_UNROLL * 256) load(i0);
+#pragma unroll
+    for (int u = 0; u < PC_UNROLL; ++u) {
+      const int64_t e = i0 + u * 256 + tid;
+      if (e < end) sorted_event(e, bv[u], bp[u], E, B, offsets, order, dst_rows);
+    }
+  }
 }
+
+// 2) The rest of the plan in one launch, up to PP_MAX_B samples and PP_MAX_COUNTS counts: every workgroup
+// sums the counts of all chunks (its base within each sample, and the samples' offsets) by itself,
+// then its wavefronts rank a quarter of the chunk each, in order.  A scan launch of its own between the
+// count and the ranking cost 24 us at 83 chunks x 256 samples (one workgroup, one dependent load per
+// chunk) and the ranking by one wavefront per chunk 15; this 8 us.  Past the limits (the counts are
+// read once per chunk) the two launches below take over.
+constexpr int PP_MAX_B = 1024;
+constexpr int64_t PP_MAX_COUNTS = 1 << 17;
+constexpr int64_t PP_MAX_E = 1ll << 30;  // rows in 32 bits
+constexpr int PP_WAVES = 4, PP_UNROLL = 4;
+
+__global__ __launch_bounds__(256) void pack_place_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx, int64_t E,
+                                                         int B, int64_t C, int nchunks,
+                                                         const int* __restrict__ counts,
+                                                         int64_t* __restrict__ offsets, int64_t* __restrict__ order,
+                                                         int64_t* __restrict__ dst_rows, int64_t* __restrict__ rank,
+                                                         int32_t* __restrict__ err, int32_t* __restrict__ ident,
+                                                         const int* __restrict__ status) {
+  __shared__ int tot[PP_MAX_B], pre[PP_MAX_B], first[PP_MAX_B];
+  __shared__ int next[PP_WAVES][PP_MAX_B];
+  __shared__ int wsum[PP_WAVES];
+  __shared__ int sorted_flag;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, chunk = blockIdx.x;
+  const bool head = chunk == 0;
+  // this wavefront's events of the first round (all of them up to 1024 per chunk)
+  const int64_t CW = cdiv(C / 64, PP_WAVES) * 64;
+  const int64_t beg = (int64_t)chunk * C + w * CW, end = min(min(E, (int64_t)(chunk + 1) * C), beg + CW);
+  int64_t bv[PP_UNROLL];
+  auto load = [&](int64_t i0) {
+#pragma unroll
+    for (int u = 0; u < PP_UNROLL; ++u) {
+      const int64_t e = i0 + u * 64 + lane;
+      bv[u] = e < end ? bidx[e * s_bidx] : -2;  // -2: no event
+    }
+  };
+  load(beg);
+  if (ranges_sorted(status, nchunks, &sorted_flag)) {
+    if (head && ident && tid == 0) *ident = 1;
+    return;
+  }
+  for (int b = tid; b < B; b += 256) {
+    tot[b] = pre[b] = 0;
+#pragma unroll
+    for (int v = 0; v < PP_WAVES; ++v) next[v][b] = 0;
+  }
+  __syncthreads();
+
+  // totals per sample and those of the chunks before this one: neighbouring threads take
+  // neighbouring samples, with few samples several threads share one
+  const int seg = B < 256 ? 256 / B : 1;
+  for (int b0 = 0; b0 < B; b0 += 256) {
+    const int b = seg > 1 ? tid % B : b0 + tid, s0 = seg > 1 ? tid / B : 0;
+    if (b >= B || s0 >= seg) continue;
+    int t = 0, p = 0;
+    constexpr int U = 16;  // loads in flight
+    for (int c0 = s0; c0 < nchunks; c0 += U * seg) {
+      int v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = c0 + u * seg;
+        v[u] = c < nchunks ? counts[(int64_t)c * B + b] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        t += v[u];
+        if (c0 + u * seg < chunk) p += v[u];
+      }
+    }
+    if (seg > 1) {
+      atomicAdd(&tot[b], t);
+      atomicAdd(&pre[b], p);
+    } else {
+      tot[b] = t;
+      pre[b] = p;
+    }
+  }
+  // and each wavefront's own counts
+  const int bits = sample_bits(B);
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  bool bad = false;
+  for (int64_t i0 = beg; i0 < end; i0 += PP_UNROLL * 64) {
+    if (i0 > beg) load(i0);
+#pragma unroll
+    for (int u = 0; u < PP_UNROLL; ++u) {
+      const int64_t b = bv[u];
+      const bool valid = b >= 0 && b < B;
+      if (!valid && i0 + u * 64 + lane < end) bad = true;
+      const uint64_t same = same_sample_lanes((int)b, valid, bits);
+      if (valid && (same & lt_mask) == 0) next[w][b] += (int)__popcll(same);
+    }
+  }
+  if (bad && err) atomicOr(err, ERR_BATCH_INDEX);
+  __syncthreads();
+
+  // exclusive scan of the totals over the samples: PP_MAX_B / 256 consecutive ones per thread
+  constexpr int PER = PP_MAX_B / 256;
+  int local = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) local += tid * PER + i < B ? tot[tid * PER + i] : 0;
+  int incl = local;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += y;
+  }
+  if (lane == 63) wsum[w] = incl;
+  __syncthreads();
+  int run = incl - local;
+  for (int v = 0; v < w; ++v) run += wsum[v];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int b = tid * PER + i;
+    if (b < B) {
+      first[b] = run;
+      if (head) offsets[b] = run;
+      int at = run + pre[b];
+#pragma unroll
+      for (int v = 0; v < PP_WAVES; ++v) {
+        const int c = next[v][b];
+        next[v][b] = at;
+        at += c;
+      }
+      run += tot[b];
+    }
+  }
+  if (head && tid == 255) {
+    offsets[B] = run;
+    if (ident) *ident = 0;  // this plan always writes `order`
+  }
+  __syncthreads();
+
+  // in-order ranking; only this wave touches its row of `next`
+  for (int64_t i0 = beg; i0 < end; i0 += PP_UNROLL * 64) {
+    if (CW > PP_UNROLL * 64) load(i0);
+#pragma unroll
+    for (int u = 0; u < PP_UNROLL; ++u) {
+      const int64_t i = i0 + u * 64 + lane, b = bv[u];
+      const bool valid = b >= 0 && b < B;
+      const uint64_t same = same_sample_lanes((int)b, valid, bits);
+      if (valid) {
+        // all lanes of a sample read its word before its lowest lane advances it (one
+        // wavefront's LDS operations complete in program order)
+        const int row0 = next[w][b];
+        const int row = row0 + (int)__popcll(same & lt_mask);
+        order[row] = i;
+        if (dst_rows) dst_rows[i] = row;
+        if (rank) rank[i] = row - first[b];
+        if ((same & lt_mask) == 0) next[w][b] = row0 + (int)__popcll(same);
+      }
+    }
+  }
+}
+
+// 2b) exclusive scan over chunks per sample (in place; SCAN_UNROLL loads in flight), then over samples.
+__global__ __launch_bounds__(1024) void pack_scan_kernel(int* __restrict__ counts, int nchunks, int B,
+                                                          int64_t* __restrict__ offsets, int32_t* __restrict__ ident,
+                                                          const int* __restrict__ status, int n_status) {
+  __shared__ int64_t part[1024];
+  __shared__ int totals[PACK_MAX_B];
+  __shared__ int sorted_flag;
+  const int tid = threadIdx.x;
+  if (ranges_sorted(status, n_status, &sorted_flag)) {
+    if (ident && tid == 0) *ident = 1;
+    return;
+  }
+  for (int b = tid; b < B; b += blockDim.x) {
+    constexpr int SCAN_UNROLL = 16;
+    int run = 0;
+    for (int c0 = 0; c0 < nchunks; c0 += SCAN_UNROLL) {
+      int t[SCAN_UNROLL];
+#pragma unroll
+      for (int u = 0; u < SCAN_UNROLL; ++u) t[u] = c0 + u < nchunks ? counts[(int64_t)(c0 + u) * B + b] : 0;
+#pragma unroll
+      for (int u = 0; u < SCAN_UNROLL; ++u) {
+        if (c0 + u < nchunks) counts[(int64_t)(c0 + u) * B + b] = run;
+        run += t[u];
+      }
+    }
+    totals[b] = run;
+  }
+  __syncthreads();
+  // each thread owns a contiguous span of samples
+  const int per = (B + blockDim.x - 1) / blockDim.x;
+  const int b0 = tid * per;
+  int64_t local = 0;
+  for (int b = b0; b < min(B, b0 + per); ++b) local += totals[b];
+  part[tid] = local;
+  __syncthreads();
+  // Hillis-Steele inclusive scan of the 1024 partials
+  for (int off = 1; off < (int)blockDim.x; off <<= 1) {
+    int64_t v = (tid >= off) ? part[tid - off] : 0;
+    __syncthreads();
+    part[tid] += v;
+    __syncthreads();
+  }
+  int64_t run = part[tid] - local;  // exclusive prefix of this span
+  for (int b = b0; b < min(B, b0 + per); ++b) {
+    offsets[b] = run;
+    run += totals[b];
+  }
+  if (tid == blockDim.x - 1) offsets[B] = part[tid];
+  if (ident && tid == 0) *ident = 0;  // this plan always writes `order`
+}
+
+// 3b) in-order ranking inside each chunk: one wavefront walks its chunk 64 events
+//    at a time; lanes holding the same sample are ranked by lane order.
+__global__ __launch_bounds__(64) void pack_rank_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx, int64_t E,
+                                                        int B, int64_t C, const int* __restrict__ chunk_base,
+                                                        const int64_t* __restrict__ offsets,
+                                                        int64_t* __restrict__ order, int64_t* __restrict__ dst_rows,
+                                                        int64_t* __restrict__ rank, int32_t* __restrict__ err,
+                                                        const int* __restrict__ status, int n_status) {
+  __shared__ int64_t next[PACK_MAX_B];
+  __shared__ int sorted_flag;
+  if (ranges_sorted(status, n_status, &sorted_flag)) return;
+  const int chunk = blockIdx.x;
+  const int lane = threadIdx.x;
+  for (int b = lane; b < B; b += 64) next[b] = offsets[b] + chunk_base[(int64_t)chunk * B + b];
+  __syncthreads();
+  const int64_t beg = (int64_t)chunk * C;
+  const int64_t end = min(E, beg + C);
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const int bits = sample_bits(B);
+  for (int64_t base = beg; base < end; base += 64) {
+    const int64_t i = base + lane;
+    int64_t b = -1;
+    if (i < end) {
+      b = bidx[i * s_bidx];
+      if (b < 0 || b >= B) {
+        b = -1;
+        if (err) atomicOr(err, ERR_BATCH_INDEX);
+      }
+    }
+    const uint64_t same = same_sample_lanes((int)b, b >= 0, bits);
+    int64_t row0 = 0;
+    if (b >= 0) {
+      row0 = next[b];  // every lane of a sample reads the same word ...
+      const int64_t row = row0 + __popcll(same & lt_mask);
+      order[row] = i;
+      if (dst_rows) dst_rows[i] = row;
+      if (rank) rank[i] = row - offsets[b];
+    }
+    __syncthreads();  // single wavefront: the reads above complete before the update
+    if (b >= 0 && (same & lt_mask) == 0) next[b] = row0 + __popcll(same);  // ... and its lowest lane advances it
+    __syncthreads();
+  }
+}
+
+// Small plans (B <= 1024, E <= PS_ONE_E) in ONE launch: one workgroup of 16 waves, wave w
+// owning the contiguous event chunk w.  Per-wave histograms in LDS, the two scans
+// (over waves per sample, then over samples), then the same in-order ranking as
+// pack_rank_kernel.  Same results as the larger plans' launches.
+// Without ranks, sorted indices are recognised first and take the identity plan.  When the
+// caller asks for an identity flag, a sorted plan sets it and leaves `order` unwritten (a
+// consumer then maps row r to event r); an unsorted one clears it and writes `order`.
+constexpr int PS_WAVES = 16;
+constexpr int PS_MAX_B = 1024;
+constexpr int PS_UNROLL = 4;
+
+// One round of loads per thread.  Above that one workgroup is latency-bound (9.5 us for a sorted plan of
+// 16384 events, 60 for a shuffled one of 65536) and the plan takes the two launches above.
+constexpr int PS_ONE_UNROLL = 4;
+constexpr int64_t PS_ONE_E = 64 * PS_WAVES * PS_ONE_UNROLL;
 
 __global__ __launch_bounds__(1024) void pack_small_kernel(const int64_t* __restrict__ bidx, int64_t s_bidx, int64_t E,
                                                           int B, int64_t* __restrict__ offsets,
                                                           int64_t* __restrict__ order, int64_t* __restrict__ dst_rows,
                                                           int64_t* __restrict__ rank, int32_t* __restrict__ err,
-                                                          const int* __restrict__ status, int n_status,
                                                           bool try_sorted, int32_t* __restrict__ ident,
                                                           bool clear_err, WidenRider wr) {
   if (blockIdx.x > 0) {  // workgroup 0 is the plan; any others carry a widening rider
@@ -311,17 +471,7 @@ __global__ __launch_bounds__(1024) void pack_small_kernel(const int64_t* __restr
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   // (every OR into err below follows at least one barrier)
   if (clear_err && err && tid == 0) clear_err_word(err, &wsum[0]);
-  if (status) {  // after pack_sorted_kernel: nothing left to do when every range was sorted
-    if (tid == 0) unsorted = 0;
-    __syncthreads();
-    for (int i = tid; i < n_status; i += blockDim.x)
-      if (status[i] != 1) unsorted = 1;
-    __syncthreads();
-    if (!unsorted) {
-      if (ident && tid == 0) *ident = 1;
-      return;
-    }
-  } else if (try_sorted) {  // E <= PS_ONE_E: the sorted check here, every load issued first
+  if (try_sorted) {  // the sorted check, every load issued first
     if (tid == 0) unsorted = 0;
     __syncthreads();
     int64_t bv[PS_ONE_UNROLL];
@@ -682,8 +832,8 @@ int64_t cortex_pack_workspace_bytes(int64_t E, int64_t B) {
   if (E <= 0 || B <= 0) return 0;
   const int64_t C = pack_chunk_size(E);
   const int64_t nchunks = cdiv(E, C);
-  // per-chunk counts (three-launch plan) and one status word per sorted-check workgroup
-  const int64_t words = nchunks * B + cdiv(E, (int64_t)PS_SORTED_EV);
+  // per-chunk counts and the status words (one per 256 events keeps the size callers have known)
+  const int64_t words = nchunks * B + cdiv(E, (int64_t)256);
   return words * (int64_t)sizeof(int);
 }
 
@@ -723,64 +873,41 @@ static int pack_plan_impl(const char* who, const int64_t* batch_indices, int64_t
               (long long)need);
     return E_WORKSPACE;
   }
-  if (B <= PS_MAX_B && E <= PS_MAX_E) {
-    // without ranks, the identity plan of sorted indices first: inside the one launch up to
-    // PS_ONE_E events, above that in the wide pack_sorted_kernel (one status word per 1024
-    // events, in the workspace: cortex_pack_workspace_bytes covers them)
-    int* status = nullptr;
-    const int n_status = (int)cdiv(E, (int64_t)PS_SORTED_EV);
-    const bool one = rank == nullptr && E <= PS_ONE_E;
-    // a widening rider joins the plan's first launch
-    if (rank == nullptr && !one && workspace != nullptr && workspace_bytes >= n_status * (int64_t)sizeof(int)) {
-      status = reinterpret_cast<int*>(workspace);
-      hipLaunchKernelGGL(pack_sorted_kernel, dim3((unsigned)(n_status + wr.blocks)), dim3(PS_SORTED_EV), 0, stream,
-                         batch_indices, s_bidx, E, (int)B, offsets, identity ? nullptr : order, dst_rows, status,
-                         clear ? err_flag : nullptr, wr);
-      CORTEX_CHECK_LAUNCH("pack_sorted_kernel");
-    }
-    const WidenRider& wr_small = status ? WidenRider{} : wr;
-    hipLaunchKernelGGL(pack_small_kernel, dim3((unsigned)(1 + wr_small.blocks)), dim3(64 * PS_WAVES), 0, stream,
-                       batch_indices, s_bidx, E, (int)B, offsets, order, dst_rows, rank, err_flag, status, n_status,
-                       one, identity, clear && status == nullptr, wr_small);
+  if (B <= PS_MAX_B && E <= PS_ONE_E) {
+    // without ranks, the identity plan of sorted indices first; a widening rider joins the launch
+    hipLaunchKernelGGL(pack_small_kernel, dim3((unsigned)(1 + wr.blocks)), dim3(64 * PS_WAVES), 0, stream,
+                       batch_indices, s_bidx, E, (int)B, offsets, order, dst_rows, rank, err_flag, rank == nullptr,
+                       identity, clear, wr);
     CORTEX_CHECK_LAUNCH("pack_small_kernel");
     return OK;
   }
   const int64_t C = pack_chunk_size(E);
   const int nchunks = (int)cdiv(E, C);
   int* counts = reinterpret_cast<int*>(workspace);
-  // Without ranks, sorted indices first (the wide check, its status words after the counts):
-  // the three launches then return at once.  The check also clears the error word.
-  int* status = nullptr;
-  const int n_status = (int)cdiv(E, (int64_t)PS_SORTED_EV);
-  if (rank == nullptr) {
-    status = counts + (int64_t)nchunks * B;
-    hipLaunchKernelGGL(pack_sorted_kernel, dim3((unsigned)(n_status + wr.blocks)), dim3(PS_SORTED_EV), 0, stream,
-                       batch_indices, s_bidx, E, (int)B, offsets, identity ? nullptr : order, dst_rows, status,
-                       clear ? err_flag : nullptr, wr);
-    CORTEX_CHECK_LAUNCH("pack_sorted_kernel");
-  } else {
-    if (clear) {
-      hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(64), 0, stream, err_flag, (int64_t)1, 0);
-      CORTEX_CHECK_LAUNCH("cortex_pack_plan(clear)");
-    }
-    const int st = widen_launch(wr, stream);
-    if (st != OK) return st;
-  }
-  hipLaunchKernelGGL(pack_count_kernel, dim3(nchunks), dim3(256), 0, stream, batch_indices, s_bidx, E, (int)B, C,
-                     counts, err_flag, status, n_status);
+  // without ranks, the check for sorted indices with the counts (its status words after them); the first
+  // launch also clears the error word and carries a widening rider
+  int* status = rank == nullptr ? counts + (int64_t)nchunks * B : nullptr;
+  hipLaunchKernelGGL(pack_count_kernel, dim3((unsigned)(nchunks + wr.blocks)), dim3(256), 0, stream, batch_indices,
+                     s_bidx, E, (int)B, C, counts, offsets, identity ? nullptr : order, dst_rows, status,
+                     clear ? err_flag : nullptr, wr);
   CORTEX_CHECK_LAUNCH("pack_count_kernel");
+  if (B <= PP_MAX_B && nchunks * B <= PP_MAX_COUNTS && E <= PP_MAX_E) {
+    hipLaunchKernelGGL(pack_place_kernel, dim3(nchunks), dim3(256), 0, stream, batch_indices, s_bidx, E, (int)B, C,
+                       nchunks, counts, offsets, order, dst_rows, rank, err_flag, identity, status);
+    CORTEX_CHECK_LAUNCH("pack_place_kernel");
+    return OK;
+  }
   hipLaunchKernelGGL(pack_scan_kernel, dim3(1), dim3(1024), 0, stream, counts, nchunks, (int)B, offsets, identity,
-                     status, n_status);
+                     status, nchunks);
   CORTEX_CHECK_LAUNCH("pack_scan_kernel");
   hipLaunchKernelGGL(pack_rank_kernel, dim3(nchunks), dim3(64), 0, stream, batch_indices, s_bidx, E, (int)B, C,
-                     counts, offsets, order, dst_rows, rank, status, n_status);
+                     counts, offsets, order, dst_rows, rank, err_flag, status, nchunks);
   CORTEX_CHECK_LAUNCH("pack_rank_kernel");
   return OK;
 }
 
-// Scratch of cortex_pack_plan_noalloc: the per-chunk counts (three-launch plan) or the
-// per-range status words (wide sorted check) that cortex_pack_plan keeps in the caller's
-// workspace.  One copy per GPU, held until the process ends.  In host code `scratch`
+// Scratch of cortex_pack_plan_noalloc: the per-chunk counts and status words that
+// cortex_pack_plan keeps in the caller's workspace.  One copy per GPU, held until the process ends.  In host code `scratch`
 // only names the symbol: its device address comes from hipGetSymbolAddress, once per
 // device, and only that address is ever handed to a kernel.
 constexpr int64_t PACK_SCRATCH_BYTES = (int64_t)4 << 20;

@@ -336,3 +336,40 @@ def test_pack_plan_widen_rider(E, B, shuffle, rank):
         assert torch.equal(got[2], want[2])
     for s, d in zip(src, dst):
         assert torch.equal(d, s.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("E,B", [(4097, 1), (4097, 3), (5000, 127), (5120, 128), (6000, 255), (8191, 256), (9000, 257),
+                                 (66000, 1000), (140000, 1024), (70000, 1025), (300000, 2), (1100000, 100)])
+@pytest.mark.parametrize("kind", ["shuffled", "runs", "bad", "strided"])
+def test_pack_plan_two_launches(E, B, kind):
+    """The count + place plan past 4096 events, at the edges of its sample segments (256 / B), chunks and
+    limits (1024 samples, 2^17 counts, chunks longer than 1024 events): exactly the stable argsort."""
+    from cortex.kernels import ops
+
+    rng = np.random.default_rng(E + B)
+    b = np.sort(rng.integers(0, B, E))
+    if kind == "runs":  # sorted chunks beside one that is not
+        b[E // 2:E // 2 + 50] = rng.integers(0, B, 50)
+    else:
+        b = b[rng.permutation(E)]
+    if kind == "bad":
+        b[rng.integers(0, E, 9)] = np.array([-1, B, B + 7, -(1 << 40), 1 << 40, B, -5, B, -1])
+    t = torch.from_numpy(b.astype(np.int64)).to(DEV)
+    if kind == "strided":
+        t = torch.stack([t, torch.full_like(t, -9)], dim=1)[:, 0]
+    valid = (b >= 0) & (b < B)
+    want = np.flatnonzero(valid)[np.argsort(b[valid], kind="stable")]
+    off = np.concatenate([[0], np.cumsum(np.bincount(b[valid], minlength=B))])
+    rank_want = np.empty(E, np.int64)
+    rank_want[want] = np.arange(len(want)) - off[b[want]]
+    for with_rank in (False, True):
+        err = torch.full((1,), 0x11, dtype=torch.int32, device=DEV)
+        got = ops.pack_plan(t, B, err=err, with_rank=with_rank, identity=True, clear_err=True)
+        assert int(err.item()) == (0 if valid.all() else 2)
+        np.testing.assert_array_equal(got[0].cpu().numpy(), off)
+        sorted_ok = not with_rank and bool(valid.all() and (np.diff(b) >= 0).all())
+        assert int(got[3].item()) == int(sorted_ok)
+        if not sorted_ok:
+            np.testing.assert_array_equal(got[1].cpu().numpy()[:len(want)], want)
+        if with_rank:
+            np.testing.assert_array_equal(got[2].cpu().numpy()[valid], rank_want[valid])
