@@ -82,6 +82,11 @@ _SIGNATURES = {
         [_i64, _i64, _i64, _int, _ptr, _i64, _int, _ptr, _ptr, _ptr, _int, _int, _int, _int, _ptr, _i64, _ptr,
          _int, _ptr, _int, _int, _ptr, _i64, _i64, _int, _ptr, _i64, _ptr],
     ),
+    "cortex_linear_small": (
+        _int,
+        [_i64, _i64, _i64, _int, _ptr, _i64, _ptr, _ptr, _f32, _int, _ptr, _i64, _ptr, _ptr, _int, _ptr, _i64, _i64, _int,
+         _ptr, _i64, _ptr],
+    ),
     "cortex_norm_linear_split_workspace_bytes": (_i64, [_i64, _i64, _i64, _int]),
     "cortex_norm_linear_split": (
         _int,

@@ -697,6 +697,71 @@ def norm_linear_fused(x: torch.Tensor, w: torch.Tensor, w_scale=None, *, norm: s
     return out
 
 
+# 32 x 32 tiles up to which linear_small beats the tiled GEMM, by K (us, tiled against small): 512: 256 x 2048 9.3 / 5.0,
+# 512 x 2048 9.3 / 8.3, 768 x 2048 9.2 / 11.4; 256: 1024 x 768 5.5 / 5.1, 2048 x 768 5.7 / 8.0; 768: 256 x 3072
+# 11.8 / 8.5, 384 x 3072 12.0 / 12.3.  The K-split residual form loses later: 2048 x 512 x 512 with its LayerNorm
+# 17.2 against 8.4 + 2.6
+_SMALL_TILES = {256: 768, 512: 1024, 768: 768}
+# and for the long K of an MLP's second linear, tiles x K (its rows in fragment order; against the K-split pair of
+# launches): 1024 x 512 x 2048 15.6 / 10.4, 1536 x 512 x 2048 15.3 / 18.2, 512 x 768 x 3072 15.1 / 10.9
+_SMALL_WORK = 1200 * 1024
+_SMALL_LN_TILES = 256  # LayerNorm inside linear_small: one workgroup per CU (128 x 1536 x 512: 6.0, apart 2.5 + 4.0; twice
+# the tiles lose, 256 x 2048 x 512: 11 against 2.6 + 5.0)
+
+
+def small_linear_ok(M: int, N: int, K: int) -> bool:
+    """Whether ``linear_small`` is the faster form of an (M, K) x (N, K) bf16 linear."""
+    if M < 1 or N % 32:
+        return False
+    tiles = ceil_div(M, 32) * (N // 32)
+    if K in _SMALL_TILES:
+        return tiles <= _SMALL_TILES[K]
+    return K in (1024, 2048, 3072) and tiles * K <= _SMALL_WORK
+
+
+def small_mlp_ok(M: int, hidden: int, D: int) -> bool:
+    """Whether an MLP's two linears run as ``linear_small`` (the hidden rows in fragment order): the second's
+    gain outweighs the first's loss up to 1536 tiles of it (768 x (512 -> 2048 -> 512): 24.1 -> 19.4 us, 1024:
+    25.1 -> 24.9)."""
+    return (D in _SMALL_TILES and hidden % 32 == 0 and M >= 1 and ceil_div(M, 32) * (hidden // 32) <= 1536
+            and small_linear_ok(M, D, hidden))
+
+
+def small_ln_ok(M: int, N: int) -> bool:
+    """Whether ``linear_small`` should apply the LayerNorm of its rows itself."""
+    return ceil_div(M, 32) * ceil_div(N, 32) <= _SMALL_LN_TILES
+
+
+def linear_small(x: torch.Tensor, weight: torch.Tensor, weight_scale=None, bias=None, *, ln=None,
+                 act: str | None = None, residual: torch.Tensor | None = None, res_rows: int = 0,
+                 out_dtype: torch.dtype = torch.bfloat16, out: torch.Tensor | None = None, rows: int | None = None,
+                 out_frag: bool = False) -> torch.Tensor:
+    """``act(a @ (weight * scale)^T + bias) + residual`` for few rows in one launch
+    (``cortex_linear_small``): ``a`` = ``x`` (M, K) bf16, or with ``ln`` = ``(weight, bias, eps)``
+    the LayerNorm of fp32 ``x`` rounded to bf16; the weight as bf16 in fragment order (``frag_weight``) or
+    as (N, K) int8 rows (widened in the kernel, the same results).
+    ``out_frag``: the bf16 result in fragment order, in a buffer of M rounded up to 16 rows, which a
+    later call takes as ``x`` with ``rows`` = M.  See ``small_linear_ok``."""
+    dev = nat.require_gpu(x, weight, weight_scale, bias, residual, out, what="linear_small")
+    x_frag = rows is not None
+    K = x.shape[1]
+    M = rows if x_frag else x.shape[0]
+    N = weight.shape[0]
+    if weight.shape[1] != K:
+        raise ValueError(f"inner dims differ: x has K={K}, weight has K={weight.shape[1]}")
+    if out is None:
+        out = torch.empty((ceil_div(M, 16) * 16 if out_frag else M, N), dtype=out_dtype, device=dev)
+    g, b, eps = ln if ln is not None else (None, None, 0.0)
+    nat.call("cortex_linear_small", M, N, K, nat.BF16_FRAG if x_frag else nat.code(x.dtype), nat.ptr(x),
+             x.stride(0) if x.shape[0] > 1 else K, nat.ptr(g), nat.ptr(b), float(eps),
+             nat.I8 if weight.dtype == torch.int8 else nat.BF16_FRAG, nat.ptr(weight), weight.stride(0),
+             nat.ptr(weight_scale), nat.ptr(bias), ACT[act], nat.ptr(residual),
+             residual.stride(0) if residual is not None and residual.shape[0] > 1 else N, int(res_rows),
+             nat.BF16_FRAG if out_frag else nat.code(out.dtype), nat.ptr(out), out.stride(0) if M > 1 else N,
+             nat.stream_of(dev))
+    return out
+
+
 def norm_linear(x: torch.Tensor, *, weight: torch.Tensor | None = None, weight_int8: torch.Tensor | None = None,
                 weight_scale: torch.Tensor | None = None, w_layout: str = "nk", norm: str | None = None,
                 gamma=None, beta=None, eps: float = 1e-5, stats=None, bias=None, act: str | None = None,

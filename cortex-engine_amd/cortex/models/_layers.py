@@ -367,6 +367,36 @@ def linear_residual_ln(lin: nn.Module, a: torch.Tensor, residual: torch.Tensor, 
                                   out=out, xq_scale=xq_scale)
 
 
+def small_ok(lin: nn.Module, x: torch.Tensor, compute: torch.dtype, norm: nn.LayerNorm | None = None) -> bool:
+    """Whether ``lin`` (after ``norm``) can run as ``ops.linear_small`` on rows of ``x``, sizes aside: bf16
+    compute, no calibration hooks, fp32 parameters."""
+    if compute != torch.bfloat16 or lin._forward_pre_hooks or (norm is not None and norm._forward_pre_hooks):
+        return False
+    if hasattr(lin, "weight_int8") and INT8_WEIGHTS != "image":
+        q = lin.weight_int8
+        if q.dim() != 2 or q.stride(1) != 1 or q.stride(0) % 8 or q.data_ptr() % 8:
+            return False
+    if lin.bias is not None and lin.bias.dtype != torch.float32:
+        return False
+    return x.dtype == torch.bfloat16 if norm is None else ln_rows_ok(x, norm)
+
+
+def small_linear(lin: nn.Module, x: torch.Tensor, norm: nn.LayerNorm | None = None, **kw) -> torch.Tensor:
+    """``lin(norm(x))`` on rows ``x`` (M, K) as ``ops.linear_small`` (see ``small_ok``); the LayerNorm in the same
+    launch where that is the faster form, else one row kernel before it.  The weight is the
+    fragment-order image, or in the INT8-resident modes the int8 rows themselves (bit-identical)."""
+    quant = hasattr(lin, "weight_int8")
+    scale = lin.weight_scale if quant else None
+    w = lin.weight_int8 if quant and INT8_WEIGHTS != "image" else frag_image(lin)
+    ln = None
+    if norm is not None:
+        if ops.small_ln_ok(x.shape[0], w.shape[0]) and x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0:
+            ln = ln_params(norm)
+        else:
+            x = normalize_bf16(x, norm)
+    return ops.linear_small(x, w, scale, lin.bias, ln=ln, **kw)
+
+
 def apply_linear(lin: nn.Module, x: torch.Tensor, *, norm: nn.LayerNorm | None = None, stats=None,
                  act: str | None = None, residual: torch.Tensor | None = None, res_rows: int = 0,
                  out_dtype: torch.dtype, compute: torch.dtype, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -382,6 +412,23 @@ def apply_linear(lin: nn.Module, x: torch.Tensor, *, norm: nn.LayerNorm | None =
             hook(lin, (xin,))
         return ops.norm_linear(xin, **linear_weights(lin), act=act, residual=residual, res_rows=res_rows,
                                out_dtype=out_dtype, compute_dtype=compute, out=out)
+    if compute == torch.bfloat16 and x.shape[-1] <= 768:
+        K = x.shape[-1]
+        N = (lin.weight_int8 if hasattr(lin, "weight_int8") else lin.weight).shape[0]
+        M = x.numel() // K if K else 0
+        # (a residual in fp32 only, so is its output; long K only with rows in fragment order)
+        if (ops.small_linear_ok(M, N, K) and stats is None and small_ok(lin, x, compute, norm)
+                and out_dtype in (torch.float32, torch.bfloat16)
+                and (residual is None or (residual.dtype == out_dtype == torch.float32 and residual.dim() == 2
+                                          and residual.shape[1] == N and residual.stride(1) == 1))
+                and (out is None or (out.dtype == out_dtype and out.is_contiguous()))):
+            x2 = x.reshape(M, K)
+            if x2.data_ptr() % 16 or x2.stride(1) != 1 or x2.stride(0) % 8:
+                x2 = x2.contiguous()
+            if out is None:
+                out = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=x.device)
+            small_linear(lin, x2, norm, act=act, residual=residual, res_rows=res_rows, out=out.reshape(M, N))
+            return out
     if (residual is not None and norm is None and act is None and compute == torch.bfloat16
             and x.dtype == torch.bfloat16 and residual.dtype == torch.float32 and out_dtype == torch.float32
             and not (hasattr(lin, "weight_int8") and INT8_WEIGHTS != "image")

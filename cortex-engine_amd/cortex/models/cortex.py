@@ -29,7 +29,7 @@ from cortex.kernels import ops
 from cortex.kernels.pack import pack_events as _device_pack_events
 from cortex.models._layers import (apply_linear, batch_invariant, bf16_weight, exec_weights, fused_tokens_ok,
                                    linear_residual_ln, linear_weights, ln_params, ln_rows_ok, normalize_bf16,
-                                   residual_ln_ok, rider)
+                                   residual_ln_ok, rider, small_ok)
 from cortex.models.config import CortexConfig
 from cortex.models.perceiver import PerceiverEncoder
 from cortex.models.tokenizer import SpikeTokenizer
@@ -271,7 +271,7 @@ class CortexModel(nn.Module):
         rows, normed = tokens
         E = rows.shape[0]
         if normed:
-            kv = ops.norm_linear(rows, **exec_weights(xa.kv_proj, compute), out_dtype=compute, compute_dtype=compute)
+            kv = apply_linear(xa.kv_proj, rows, out_dtype=compute, compute=compute)
         else:
             kv = apply_linear(xa.kv_proj, rows, norm=xa.norm_kv, out_dtype=compute, compute=compute)  # (E, 2D)
         q = xa.project_queries(enc.latents, compute)  # (L, D), shared by every sample
@@ -279,7 +279,8 @@ class CortexModel(nn.Module):
         ops.attention(ops.heads_view(q, 1, L, H), ops.heads_view(kv, 1, E, H, 0, D),
                       ops.heads_view(kv, 1, E, H, D, D), kv_offsets=offsets, out=o, batch=B)
         first = enc.self_attn_blocks[0] if len(enc.self_attn_blocks) else None
-        if first is not None and residual_ln_ok(xa.out_proj, first.norm_attn, first.qkv_proj, enc.latents, compute):
+        few = ops.small_linear_ok(B * L, D, D) and small_ok(xa.out_proj, o_buf, compute)
+        if not few and first is not None and residual_ln_ok(xa.out_proj, first.norm_attn, first.qkv_proj, enc.latents, compute):
             # latents + out_proj(attn) and the first block's norm_attn in one launch
             return linear_residual_ln(xa.out_proj, o_buf, enc.latents, first.norm_attn, res_rows=L,
                                       out=torch.empty(B * L, D, dtype=torch.float32, device=kv.device))

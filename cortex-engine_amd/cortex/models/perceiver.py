@@ -17,7 +17,7 @@ from torch import nn
 from cortex.kernels import ops
 from cortex.models import _layers
 from cortex.models._layers import (apply_linear, batch_invariant, build_weight_window, exec_weights, fused_weight,
-                                   linear_residual_ln, ln_rows_ok, normalize_bf16, residual_ln_ok, rider)
+                                   linear_residual_ln, ln_rows_ok, normalize_bf16, residual_ln_ok, rider, small_linear, small_ok)
 from cortex.models.config import CortexConfig
 
 
@@ -93,7 +93,8 @@ class SelfAttentionBlock(nn.Module):
         rows when the producer of ``x`` already wrote it.
 
         With bf16 compute, ``x + out_proj(attn)`` and ``norm_mlp`` of the result run as one
-        kernel (``ops.linear_residual_ln``); the LayerNorm'd rows feed ``mlp.0`` directly.
+        kernel (``ops.linear_residual_ln``); the LayerNorm'd rows feed ``mlp.0`` directly.  With
+        few rows every linear is one ``ops.linear_small`` launch.
         """
         compute = self.config.compute_dtype
         D = x.shape[1]
@@ -101,15 +102,19 @@ class SelfAttentionBlock(nn.Module):
         w8 = self._w8a8(x, compute)
         if w8 is not None and w8[2] is not None and self._fused_attention_ok(x, length):
             return self._forward_rows_w8a8(x, batch, length, inplace, w8)
-        if self._fused_attention_ok(x, length):
+        M = batch * length
+        fused = self._fused_attention_ok(x, length)
+        few = w8 is None and ops.small_linear_ok(M, D, D)  # (no larger linear of the block is, past this)
+        if fused and few and self._small_attention_ok(x, M):
+            fused = False  # few rows: the projection over 32 x 32 tiles and the attention on their own
+        if fused:
             # qkv projection + attention per (head, sample) on chip: qkv never reaches HBM
             if xn is None:  # this block's weights widen into their window in the same launch
                 xn = normalize_bf16(x, self.norm_attn, widen=rider(self, rows=x.numel() // x.shape[-1]))
             o_buf = ops.qkv_attention(xn, *fused_weight(self.qkv_proj, rows=batch * length), batch, length, H)
         else:
             if xn is not None:
-                qkv = ops.norm_linear(xn, **exec_weights(self.qkv_proj, compute), out_dtype=compute,
-                                      compute_dtype=compute)
+                qkv = apply_linear(self.qkv_proj, xn, out_dtype=compute, compute=compute)
             else:
                 qkv = apply_linear(self.qkv_proj, x, norm=self.norm_attn, out_dtype=compute, compute=compute)
             o_buf, o = ops.merge_heads_out(batch, length, H, D // H, compute, x.device)
@@ -123,16 +128,34 @@ class SelfAttentionBlock(nn.Module):
             hq = ops.linear_w8a8(xq, w8[0], up.weight_int8, up.weight_scale, up.bias, act="gelu",
                                  out_dtype=torch.int8, out_scale=w8[1])
             return ops.linear_w8a8(hq, w8[1], down.weight_int8, down.weight_scale, down.bias, residual=x, out=x)
-        if residual_ln_ok(self.out_proj, self.norm_mlp, self.mlp[0], x, compute):
+        hn = None
+        if few and small_ok(self.out_proj, o_buf, compute):
+            x = apply_linear(self.out_proj, o_buf, residual=x, out_dtype=x.dtype, compute=compute,
+                             out=x if inplace else None)
+        elif residual_ln_ok(self.out_proj, self.norm_mlp, self.mlp[0], x, compute):
             x, hn = linear_residual_ln(self.out_proj, o_buf, x, self.norm_mlp, out=x if inplace else None)
-            h = ops.norm_linear(hn, **exec_weights(self.mlp[0], compute), act="gelu", out_dtype=compute,
-                                compute_dtype=compute)
         else:
             x = apply_linear(self.out_proj, o_buf, residual=x, out_dtype=x.dtype, compute=compute,
                              out=x if inplace else None)
-            h = apply_linear(self.mlp[0], x, norm=self.norm_mlp, act="gelu", out_dtype=compute, compute=compute)
-        return apply_linear(self.mlp[2], h, residual=x, out_dtype=x.dtype, compute=compute,
-                            out=x if inplace else None)
+        up, down = self.mlp[0], self.mlp[2]
+        if (few and ops.small_mlp_ok(M, int(D * self.config.mlp_ratio), D) and small_ok(up, x, compute, self.norm_mlp)
+                and small_ok(down, o_buf, compute)):
+            h = small_linear(up, x if hn is None else hn, self.norm_mlp if hn is None else None, act="gelu",
+                             out_frag=True)
+            return small_linear(down, h, residual=x, rows=M, out_dtype=x.dtype, out=x if inplace else None)
+        if hn is not None:
+            h = ops.norm_linear(hn, **exec_weights(up, compute), act="gelu", out_dtype=compute, compute_dtype=compute)
+        else:
+            h = apply_linear(up, x, norm=self.norm_mlp, act="gelu", out_dtype=compute, compute=compute)
+        return apply_linear(down, h, residual=x, out_dtype=x.dtype, compute=compute, out=x if inplace else None)
+
+    def _small_attention_ok(self, x: torch.Tensor, M: int) -> bool:
+        """Whether the QKV projection (``linear_small``) and the attention as two launches beat the fused
+        kernel, whose few workgroups (one per head and sample) each take 10 to 16 us: D 512, L 256, B 1 / 2:
+        16.1 / 16.4 against 11.8 / 14.0 us; D 256, L 128, B 4 / 8: 10.2 / 10.2 against 8.9 / 10.4."""
+        D = x.shape[1]
+        return (ops.ceil_div(M, 32) * (3 * D // 32) <= (512 if D == 256 else 1024)
+                and small_ok(self.qkv_proj, x, torch.bfloat16, self.norm_attn))
 
     def _w8a8(self, x: torch.Tensor, compute: torch.dtype) -> tuple | None:
         """``(s_up, s_down, attn)`` activation scales when this block runs its MLP as W8A8

@@ -253,6 +253,20 @@ int cortex_norm_linear(int64_t M, int64_t N, int64_t K, int x_dtype, const void*
                        int64_t ld_res, int64_t res_rows, int out_dtype, void* out, int64_t ld_out,
                        hipStream_t stream);
 
+/* A bf16 linear with few rows in one launch (the chains of SelfAttentionBlock and
+ * CrossAttentionBlock, cortex/models/perceiver.py:67-68,113-125, at one to a few samples):
+ *   out = act((a . w^T) * w_scale + bias) + residual[m % res_rows]
+ * a: bf16 rows (gamma NULL; x_dtype 1, or 7 for rows in fragment order), or bf16(LayerNorm(x)) of fp32 rows
+ * (x_dtype 0, gamma and beta given, fp32), its statistics computed by the call.  K 256, 512, 768 or 1024,
+ * without LayerNorm also 2048 or 3072; w the (N, K) weight, w_dtype 7 for bf16 in fragment order
+ * (cortex_frag_weight; ld_w ignored) or 3 for int8 rows (8-byte aligned, the same results), N a multiple of 16; rows 16-byte aligned; w_scale, bias, residual optional fp32; act 0 or 1 (erf-GELU); out
+ * fp32 (0, may be residual), bf16 (1) or bf16 in fragment order (7: as cortex_frag_weight's, M rounded up
+ * to 16 rows, N a multiple of 32; the row strides are ignored); res_rows 0 means M. */
+int cortex_linear_small(int64_t M, int64_t N, int64_t K, int x_dtype, const void* x, int64_t ld_x,
+                        const float* gamma, const float* beta, float eps, int w_dtype, const void* w, int64_t ld_w,
+                        const float* w_scale, const float* bias, int act, const float* residual, int64_t ld_res,
+                        int64_t res_rows, int out_dtype, void* out, int64_t ld_out, hipStream_t stream);
+
 /* The fp32-compute form of cortex_norm_linear on the bf16 matrix cores (the fp32 rows of
  * cortex/kernels/fused_rmsnorm.py:239-301 and of QuantizedLinear, calibrate.py:225-228): every
  * fp32 operand as the exact sum of three bf16 parts, products and sums in fp32 (an int8 weight is

@@ -1,0 +1,96 @@
+"""The few-row bf16 linear (gemm_small.hip) against 64-bit products of the same bf16 operands.
+
+Row counts around its 32-row tiles and 16-row fragment blocks, every K it takes, both operand and output
+orders.  fp32 outputs: at most K / 32 + 16 accumulations of 2^-24 of sum |a| |w|; bf16 outputs and the
+LayerNorm'd operand add half a bf16 step (2^-9) each.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _unfrag(t: torch.Tensor, rows: int) -> torch.Tensor:
+    """Rows of a fragment-order (R, N) tensor (R a multiple of 16)."""
+    R, N = t.shape
+    return t.reshape(R // 16, N // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(R, N)[:rows]
+
+
+def _case(M, N, K, seed):
+    g = torch.Generator(DEV).manual_seed(seed)
+    x = torch.randn(M, K, generator=g, device=DEV)
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
+    s = torch.rand(N, generator=g, device=DEV) + 0.5
+    b = torch.randn(N, generator=g, device=DEV)
+    return g, x, w, s, b
+
+
+@pytest.mark.parametrize("K", [256, 512, 768, 1024, 2048, 3072])
+@pytest.mark.parametrize("M,N", [(1, 32), (15, 64), (16, 96), (17, 32), (33, 160), (129, 64)])
+def test_bf16_rows_residual_and_orders(M, N, K):
+    from cortex.kernels import ops
+
+    g, x, w, s, b = _case(M, N, K, M + N + K)
+    xb, wf = x.bfloat16(), ops.frag_weight(w)
+    res = torch.randn(7, N, generator=g, device=DEV)
+    y = xb.double() @ w.double().t().contiguous() * s.double() + b.double()
+    acc = (K / 32 + 16) * 2.0 ** -24 * (xb.double().abs() @ w.double().abs().t().contiguous() * s.double() + y.abs() + 8)
+    want = y + res.double().repeat(M // 7 + 1, 1)[:M]
+    got = ops.linear_small(xb, wf, s, b, residual=res, res_rows=7, out_dtype=torch.float32)
+    assert ((got - want).abs() <= acc).all()
+    buf = torch.randn(M, N, generator=g, device=DEV)
+    want = buf.double() + y
+    ops.linear_small(xb, wf, s, b, residual=buf, out=buf)
+    assert ((buf - want).abs() <= acc).all()
+    q, qs = ops.quantize_int8(w.float())  # int8 rows: bit for bit their bf16 image
+    a8 = ops.linear_small(xb, q, qs, b, act="gelu")
+    assert torch.equal(a8, ops.linear_small(xb, ops.frag_weight(q), qs, b, act="gelu"))
+    # GELU to bf16 rows, the same in fragment order, and that order as the operand of the next linear
+    act = torch.nn.functional.gelu(y)
+    rows = ops.linear_small(xb, wf, s, b, act="gelu")
+    assert ((rows.double() - act).abs() <= 1.13 * acc + 2.0 ** -8 * act.abs() + 1e-6).all()
+    h = ops.linear_small(xb, wf, s, b, act="gelu", out_frag=True)
+    assert h.shape[0] % 16 == 0 and torch.equal(_unfrag(h, M), rows)
+    xf = torch.zeros((M + 15) // 16 * 16, K, dtype=torch.bfloat16, device=DEV)
+    xf[:M] = xb
+    again = ops.linear_small(ops.frag_weight(xf), wf, s, b, rows=M, out_dtype=torch.float32)
+    assert torch.equal(again, ops.linear_small(xb, wf, s, b, out_dtype=torch.float32))
+
+
+@pytest.mark.parametrize("K", [256, 512, 768, 1024])
+@pytest.mark.parametrize("M", [1, 31, 64, 100])
+def test_layer_norm_inside(M, K):
+    from cortex.kernels import ops
+
+    g, x, w, s, _ = _case(M, 96, K, M + K)
+    x = torch.cat([x * 3 + 1, x], 1)[:, :K]  # rows at a stride of 2 K
+    gm, bt = 1 + 0.1 * torch.randn(K, generator=g, device=DEV), 0.1 * torch.randn(K, generator=g, device=DEV)
+    a = torch.nn.functional.layer_norm(x.double(), (K,), gm.double(), bt.double(), 1e-5)
+    want = a @ w.double().t().contiguous() * s.double()
+    mag = (a.abs() + 0.1) @ w.double().abs().t().contiguous() * s.double()
+    got = ops.linear_small(x, ops.frag_weight(w), s, ln=(gm, bt, 1e-5), out_dtype=torch.float32)
+    assert ((got - want).abs() <= (2.0 ** -9 + (K / 32 + 40) * 2.0 ** -24) * mag).all()
+    assert ((got - want).norm() <= 2.0 ** -9 * want.norm())
+
+
+@pytest.mark.parametrize("model", ["xs", "s", "m"])
+@pytest.mark.parametrize("batch", [1, 2, 3, 5, 9])
+def test_block_around_the_few_row_rule(model, batch):
+    """A block on either side of the few-row rules against the same block in fp32 compute."""
+    from cortex.models import config
+    from cortex.models.perceiver import SelfAttentionBlock
+
+    cfg = getattr(config, "CORTEX_" + model.upper())
+    torch.manual_seed(0)
+    blk = SelfAttentionBlock(cfg).to(DEV).eval()
+    ref = SelfAttentionBlock(cfg.model_copy(update={"dtype": "float32"})).to(DEV).eval()
+    ref.load_state_dict(blk.state_dict())
+    x = torch.randn(batch, cfg.num_latents, cfg.latent_dim, device=DEV)
+    with torch.no_grad():
+        got, want = blk(x), ref(x)
+    # (bf16 operands, and a float weight rounded to bf16: a few bf16 steps of the branches' size)
+    assert ((got - want).norm() <= 1e-2 * (want - x).norm())
