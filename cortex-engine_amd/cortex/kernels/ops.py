@@ -284,7 +284,7 @@ def ln_rows(x: torch.Tensor, ln1, ln2=None, out_bf16: bool = True, out_f32: bool
     Returns the bf16 and/or fp32 result(s).  ``widen``: (int8, bf16) weight pairs widened by
     extra workgroups of the same launch (``widen_int8``)."""
     dev = nat.require_gpu(x, what="ln_rows")
-    x2 = _row_major_2d(x.reshape(-1, x.shape[-1]))
+    x2 = _row_major_2d(x if x.dim() == 2 else x.reshape(-1, x.shape[-1]))
     M, K = x2.shape
     ob = torch.empty((M, K), dtype=torch.bfloat16, device=dev) if out_bf16 else None
     of = torch.empty((M, K), dtype=torch.float32, device=dev) if out_f32 else None
@@ -762,6 +762,33 @@ def linear_small(x: torch.Tensor, weight: torch.Tensor, weight_scale=None, bias=
     return out
 
 
+def _plain_bf16_linear(x, weight, weight_scale, bias, act, residual, res_rows, out_dtype, out) -> torch.Tensor:
+    """``norm_linear`` of contiguous bf16 rows and weight without a norm: the same launches, with the
+    questions that contiguous operands answer left out (half of a block's time on the host)."""
+    dev = nat.require_gpu(x, weight, weight_scale, bias, residual, out, what="norm_linear")
+    N, K = weight.shape
+    M = x.numel() // K if K else 0
+    if out is None:
+        out = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=dev)
+    elif out.numel() != M * N:
+        raise ValueError("out must be row-major contiguous over its last dim")
+    wp, xp, op, sp, bp, rp = (nat.ptr(t) for t in (weight, x, out, weight_scale, bias, residual))
+    if (residual is not None and not ACT[act] and residual.dtype == out.dtype == torch.float32
+            and (bias is None or bias.dtype == torch.float32)
+            and not ((wp | xp | op | (sp or 0) | (bp or 0) | rp) & 15) and not (K & 7 or N & 3)):
+        splits = splitk_splits(M, N, K, dev)
+        if splits:  # few rows: K split across workgroups, slabs summed in order
+            ws_t = torch.empty(nat.load().cortex_splitk_workspace_bytes(M, N, splits), dtype=torch.uint8, device=dev)
+            nat.call("cortex_linear_residual_splitk", M, N, K, xp, K, wp, K, sp, bp, rp, N, int(res_rows), op, N, splits,
+                     nat.ptr(ws_t), ws_t.numel(), nat.stream_of(dev))
+            return out
+    nat.call("cortex_norm_linear", M, N, K, nat.BF16, xp, K, 0, None, None, None, nat.F32, nat.BF16, nat.BF16, 0, wp, K,
+             sp, nat.code(bias.dtype) if bias is not None else nat.F32, bp, ACT[act],
+             nat.code(residual.dtype) if residual is not None else nat.F32, rp, N if residual is not None else 0,
+             int(res_rows), nat.code(out.dtype), op, N, nat.stream_of(dev))
+    return out
+
+
 def norm_linear(x: torch.Tensor, *, weight: torch.Tensor | None = None, weight_int8: torch.Tensor | None = None,
                 weight_scale: torch.Tensor | None = None, w_layout: str = "nk", norm: str | None = None,
                 gamma=None, beta=None, eps: float = 1e-5, stats=None, bias=None, act: str | None = None,
@@ -773,6 +800,11 @@ def norm_linear(x: torch.Tensor, *, weight: torch.Tensor | None = None, weight_i
     (``'kn'``, rms_norm_linear) matrix; ``weight_int8``/``weight_scale`` is the
     QuantizedLinear form.  ``compute_dtype`` is the MFMA input dtype (bf16 or fp32).
     """
+    if (norm is None and weight is not None and weight.dtype is torch.bfloat16 and x.dtype is torch.bfloat16
+            and compute_dtype is torch.bfloat16 and w_layout == "nk" and weight_int8 is None
+            and weight.dim() == 2 and x.shape[-1] == weight.shape[1] and x.is_contiguous() and weight.is_contiguous()
+            and all(t is None or t.is_contiguous() for t in (weight_scale, residual, out))):
+        return _plain_bf16_linear(x, weight, weight_scale, bias, act, residual, res_rows, out_dtype or x.dtype, out)
     w = weight if weight is not None else weight_int8
     dev = nat.require_gpu(x, w, weight_scale, gamma, beta, bias, residual, out, what="norm_linear")
     K = x.shape[-1]
@@ -912,11 +944,11 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float
         raise ValueError("q, k, v must share a dtype")
     if q.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError(f"attention dtype {q.dtype} not supported (bfloat16 or float32)")
-    for t in (q, k, v):
-        if t.stride(-1) != 1:
-            raise ValueError("attention inputs need a contiguous last (head) dim")
-    B = q.shape[0] if batch is None else batch
-    H, Lq, Dh = q.shape[1], q.shape[2], q.shape[3]
+    (qsb, qsh, qsl, q1), (ksb, ksh, ksl, k1), (vsb, vsh, vsl, v1) = q.stride(), k.stride(), v.stride()
+    if not q1 == k1 == v1 == 1:
+        raise ValueError("attention inputs need a contiguous last (head) dim")
+    n, H, Lq, Dh = q.shape
+    B = n if batch is None else batch
     Lk = k.shape[2]
     if out is None:
         out = torch.empty((B, H, Lq, Dh), dtype=q.dtype, device=dev)
@@ -936,14 +968,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float
             raise ValueError(f"block_mask must be (n_q, n_k) or ({B}, n_q, n_k), got {tuple(block_mask.shape)}")
         n_qt, n_kt = block_mask.shape[-2], block_mask.shape[-1]
         bm_sb = block_mask.stride(0) if block_mask.dim() == 3 else 0
-    qsb = q.stride(0) if q.shape[0] > 1 else 0
+    osb, osh, osl, _ = out.stride()
     nat.call("cortex_attention", nat.code(q.dtype), B, H, Lq, Lk, Dh,
-             nat.ptr(q), qsb, q.stride(1), q.stride(2),
-             nat.ptr(k), k.stride(0), k.stride(1), k.stride(2),
-             nat.ptr(v), v.stride(0), v.stride(1), v.stride(2),
+             nat.ptr(q), qsb if n > 1 else 0, qsh, qsl, nat.ptr(k), ksb, ksh, ksl, nat.ptr(v), vsb, vsh, vsl,
              nat.ptr(kv_offsets), nat.ptr(kv_lengths), nat.ptr(key_mask), km_sb,
              nat.ptr(block_mask), bm_sb, n_qt, n_kt, int(block_l), int(block_e), s,
-             nat.ptr(out), out.stride(0), out.stride(1), out.stride(2), nat.stream_of(dev))
+             nat.ptr(out), osb, osh, osl, nat.stream_of(dev))
     return out
 
 

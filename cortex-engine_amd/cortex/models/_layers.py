@@ -321,7 +321,7 @@ def normalize_bf16(x: torch.Tensor, norm: nn.LayerNorm, norm2: nn.LayerNorm | No
                    widen: list | None = None) -> torch.Tensor:
     """``norm2(norm(x))`` (or ``norm(x)``) as bf16 rows (one launch; ``widen``: weight pairs that
     ride along, see ``WeightWindow``)."""
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if x2.data_ptr() % 16 or (x2.shape[0] > 1 and x2.stride(0) % 4) or x2.stride(-1) != 1:
         x2 = x2.contiguous()
     return ops.ln_rows(x2, ln_params(norm), ln_params(norm2) if norm2 is not None else None, widen=widen)
