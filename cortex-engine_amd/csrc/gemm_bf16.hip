@@ -554,7 +554,7 @@ int cu_count() {
 // The K loop, ring, swizzles and epilogue arithmetic are gemm_bf16_kernel's (B256x256s2,
 // interleaved W rows, 8 consecutive columns per lane; transfers from a uniform base plus a
 // 32-bit lane offset).  A tile's 256 column scales and biases travel into LDS with its first
-// stages (two buffers, by tile parity, since the next tile's arrive during this tile's
+// stages (two buffers in turn, since the next tile's arrive during this tile's
 // epilogue).  The epilogue issues exactly one 16-byte store per (row group, column group) and
 // lane -- rows past M store row M - 1's values again, computed from the clamped A rows, so the
 // duplicates are bit-identical -- so the first waits of the next tile count them exactly.
@@ -569,7 +569,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
   constexpr int NST = TM * NG;  // stores per lane and tile
   static_assert(S == 2 && TL::KS == 1 && TL::WAVES == 8, "two-stage ring, one K group, 8 wavefronts");
   static_assert(PER + NST < 64, "vmcnt range");
-  constexpr int PAR = TL::LDS;  // column parameters: [parity][scale 256 | bias 256] floats
+  constexpr int PAR = TL::LDS;  // column parameters: [turn][scale 256 | bias 256] floats
   __shared__ __attribute__((aligned(1024))) unsigned char smem[TL::LDS + 2 * 2 * BN * 4];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
   const int wu = __builtin_amdgcn_readfirstlane(wid);
   auto a_stage = [&](int s) __attribute__((always_inline)) { return smem + s * TL::A_STAGE; };
   auto w_stage = [&](int s) __attribute__((always_inline)) { return smem + S * TL::A_STAGE + s * TL::W_STAGE; };
-  auto params = [&](int t) __attribute__((always_inline)) { return reinterpret_cast<float*>(smem + PAR) + (t & 1) * 2 * BN; };
+  auto params = [&](int turn) __attribute__((always_inline)) { return reinterpret_cast<float*>(smem + PAR) + turn * 2 * BN; };
   const int nk = K / TL::BK;
 
   // The transfer offsets (bytes from the operand bases; the host keeps both below 4 GiB) are
@@ -627,14 +627,14 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
   };
   // a tile's first stages, its column parameters ahead of them (4 bytes per lane: wavefronts
   // 0-3 the 256 scales, 4-7 the biases; null ones are never read)
-  auto prologue = [&](int t) __attribute__((always_inline)) {
+  auto prologue = [&](int t, int turn) __attribute__((always_inline)) {
     m0c = (t / gx) * BM;
     n0c = (t % gx) * BN;
     const int n0 = n0c;
     const float* src = wu < 4 ? scale : bias;
     if (src)
       lds_dma_m0<4>(src + n0 + (wu & 3) * 64, (uint32_t)(threadIdx.x & 63) * 4u,
-                    lds0 + PAR + ((t & 1) * 2 * BN + (wu < 4 ? 0 : BN) + (wu & 3) * 64) * 4);
+                    lds0 + PAR + (turn * 2 * BN + (wu < 4 ? 0 : BN) + (wu & 3) * 64) * 4);
 #pragma unroll
     for (int p = 0; p < S; ++p)
       if (p < nk) issue(p);
@@ -691,9 +691,9 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
 
   // tile t's epilogue from registers and its column parameters in LDS: one store per (row
   // group, column group) and lane
-  auto epilogue = [&](int t) __attribute__((always_inline)) {
+  auto epilogue = [&](int t, int turn) __attribute__((always_inline)) {
     const int m0 = (t / gx) * BM, n0 = (t % gx) * BN;
-    const float* sp = params(t);
+    const float* sp = params(turn);
     // row offsets in elements, 32-bit (M * ld_out * 2 < 4 GiB, checked at launch), once per tile
     uint32_t roff[TM];
 #pragma unroll
@@ -731,7 +731,10 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
   };
 
   if (t0 >= tend) return;
-  prologue(t0);
+  // the column parameters' buffer changes with every tile (not with the tile number: that advances by
+  // tstep, mostly even, and the next tile's columns would overwrite the ones in use)
+  int turn = 0;
+  prologue(t0, turn);
   bool after = false;  // the previous tile's epilogue stores are still counted by vmcnt
   for (int t = t0;; t += tstep) {
 #pragma unroll
@@ -762,8 +765,9 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
     mma(af1, wf1);
     const int next = t + tstep;
     __builtin_amdgcn_s_barrier();  // every wave is done with the ring: the next tile may refill it
-    if (next < tend) prologue(next);
-    epilogue(t);
+    if (next < tend) prologue(next, turn ^ 1);
+    epilogue(t, turn);
+    turn ^= 1;
     if (next >= tend) break;
     after = true;
   }
