@@ -48,6 +48,10 @@ int try_gemm_bf16(const GemmArgs& g, int x_dtype, int w_dtype, int w_layout, int
 // aligned rows.  Returns OK or an error status.
 int launch_res_dw(const GemmArgs& g, hipStream_t stream);
 
+// Residual GEMM on 256 x 256 tiles by four wavefronts (gemm_wide.hip): bf16 x and w, fp32 residual and output,
+// N % 256 == 0, K % 64 == 0 and long, tiles that fill the CUs.  Same return convention.
+int try_gemm_wide(const GemmArgs& g, hipStream_t stream);
+
 // K split over gridDim.z = splits workgroup slabs (gemm_bf16.hip): slab z computes
 // (x[:, zK:(z+1)K] . w[:, zK:(z+1)K]^T) * w_scale into g.out + z * M * ld_out (fp32), where
 // K = g.K is the per-slab depth (a multiple of 64) and g.x / g.w are the full rows.  No

@@ -1570,6 +1570,10 @@ int try_gemm_bf16(const GemmArgs& g, int x_dtype, int w_dtype, int w_layout, int
   // 2.647 / 5.42 ms with these.
   if (res) {
     if (g.act || g.K % 128) return 0;
+    if (!w8) {  // long K and many tiles
+      const int wide = try_gemm_wide(g, stream);
+      if (wide != 0) return wide;
+    }
     if (!w8 && g.N % 128 == 0 && cdiv(g.M, 128) * cdiv(g.N, 128) > cu_count())
       return launch<B256x128s3, ACT_NONE, true, float, bf16, bf16>(g, stream);
     return w8 ? launch<B128x128s2k2w, ACT_NONE, true, float, bf16, int8_t>(g, stream)

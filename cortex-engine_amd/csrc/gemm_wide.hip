@@ -1,10 +1,9 @@
-// bf16 GEMM on 256 x 256 tiles for gfx950, for launches of at least one such tile per CU:
+// Residual bf16 GEMM on 256 x 256 tiles for gfx950 (MLP-down with many rows):
 //
-//   y[m, n] = epi( sum_k a[m, k] w[n, k] ),  a (M, K), w (N, K) bf16 rows
-//   epi: * w_scale[n] (+ bias[n]) (-> erf-GELU) -> bf16, or (+ fp32 residual) -> fp32
+//   y[m, n] = (sum_k a[m, k] w[n, k]) * w_scale[n] (+ bias[n]) + residual[m, n],  a (M, K), w (N, K) bf16 rows, fp32 out
 //
-// What bounds it: the matrix cores (throttled by power to 1.83 PFLOP/s on random data) and, close behind, the
-// LDS: a K step of 64 writes 64 KiB into it and reads what the wavefronts need of it.  Eight wavefronts of
+// What bounds it: memory (65536 x 512 x 2048: 537 MB, 104 us at the 5.1 TB/s of a copy), the matrix cores
+// (throttled by power to 1.83 PFLOP/s on random data: 75 us) and, close behind, the LDS: a K step of 64 writes 64 KiB into it and reads what the wavefronts need of it.  Eight wavefronts of
 // 128 x 64 read 192 KiB per step of 2048 MFMA cycles, 125 bytes a cycle with the writes, all that the LDS
 // gives; four of 128 x 128 read 128 KiB, 94.  One wavefront per SIMD then has to keep its matrix core busy by
 // itself: v_mfma_f32_32x32x16_bf16 is issued at the full rate by one wavefront (16x16x32 only every 27 of its
@@ -13,8 +12,13 @@
 //
 // Persistent: a workgroup per CU walks its tiles in XCD order; after a tile's last step the next tile's two
 // stages are issued, and land while the epilogue runs.  The epilogue takes 32 rows x 64 columns of a wavefront
-// at a time through LDS of its own, so that rows are stored in whole 128-byte lines and scale, bias and
-// the GELU work on a lane's fixed eight columns.
+// at a time through LDS of its own, so that residual and output rows move in whole 256-byte pieces and a lane's
+// scale and bias columns stay the same.
+//
+// Against 256 x 128 tiles of eight wavefronts: 32768 x 512 x 2048 87.6 -> 79.1 us, 65536 x 512 x 2048 178.7 -> 160.6,
+// 36864 x 768 x 3072 225 -> 194.  (With a bf16 output and the GELU in place of the residual, K = 512, it is the
+// slower form, 205 against 216 us at 65536 x 2048 x 512: one wavefront per SIMD has nothing to overlap the
+// epilogue's arithmetic with.)
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -66,7 +70,6 @@ struct WideArgs {
   int nt, tiles;
 };
 
-template <int ACT, bool RES>
 __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(WideArgs g) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[GW_LDS];
   const int tid = threadIdx.x, lane = tid & 63, wid = wave_uniform(tid >> 6);
@@ -121,8 +124,8 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(WideArgs g) {
     for (int i = 0; i < 16; ++i) issue(i, s, s);
 
   for (;;) {
-    // scale and bias of this lane's columns: 8 of each 64-column patch (RES: 4)
-    constexpr int NC = RES ? 4 : 8, LPR = 64 / NC;  // columns per lane, lanes per row
+    // scale and bias of this lane's columns: 4 of each 64-column patch
+    constexpr int NC = 4, LPR = 64 / NC;  // columns per lane, lanes per row
     const int m0 = t / g.nt * GW_T, n0 = t % g.nt * GW_T;
     const int pc = n0 + wn * 128 + lane % LPR * NC;
     float sc[2][NC], bi[2][NC];
@@ -203,14 +206,12 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(WideArgs g) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const int mp = m0 + wm * 128 + 32 * i;
-        float4 rv[RES ? 32 / RPI : 1];
-        if constexpr (RES) {
+        float4 rv[32 / RPI];
 #pragma unroll
-          for (int x = 0; x < 32 / RPI; ++x) {
-            const int m = min(mp + x * RPI + lane / LPR, g.M - 1);
-            rv[x] = *reinterpret_cast<const float4*>(
-                g.res + (int64_t)(g.res_rows > 0 ? m % g.res_rows : m) * g.ld_res + pc + 64 * p);
-          }
+        for (int x = 0; x < 32 / RPI; ++x) {
+          const int m = min(mp + x * RPI + lane / LPR, g.M - 1);
+          rv[x] = *reinterpret_cast<const float4*>(
+              g.res + (int64_t)(g.res_rows > 0 ? m % g.res_rows : m) * g.ld_res + pc + 64 * p);
         }
         // lane: row lane % 32, columns 32 j + 8 b + 4 (lane / 32) .. +3 of the patch
 #pragma unroll
@@ -231,22 +232,10 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(WideArgs g) {
             *reinterpret_cast<f32x4*>(v + e) = *reinterpret_cast<const f32x4*>(
                 patch + r * GW_LD + ((lane % LPR * (NC / 4) + e / 4) ^ (r & 15)) * 4);
 #pragma unroll
-          for (int e = 0; e < NC; ++e) {
-            v[e] = v[e] * sc[p][e] + bi[p][e];
-            if (ACT == ACT_GELU) v[e] = gelu_erf_bf16out(v[e]);
-          }
-          if (m < g.M) {
-            if constexpr (RES) {
-              float* o = reinterpret_cast<float*>(g.out) + (int64_t)m * g.ld_out + pc + 64 * p;
-              *reinterpret_cast<float4*>(o) =
-                  make_float4(v[0] + rv[x].x, v[1] + rv[x].y, v[2] + rv[x].z, v[3] + rv[x].w);
-            } else {
-              bf16x8 h;
-#pragma unroll
-              for (int e = 0; e < 8; ++e) h[e] = (bf16)v[e];
-              *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(g.out) + (int64_t)m * g.ld_out + pc + 64 * p) = h;
-            }
-          }
+          for (int e = 0; e < NC; ++e) v[e] = v[e] * sc[p][e] + bi[p][e];
+          if (m < g.M)
+            *reinterpret_cast<float4*>(reinterpret_cast<float*>(g.out) + (int64_t)m * g.ld_out + pc + 64 * p) =
+                make_float4(v[0] + rv[x].x, v[1] + rv[x].y, v[2] + rv[x].z, v[3] + rv[x].w);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next patch overwrites it
       }
@@ -258,12 +247,12 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(WideArgs g) {
 }  // namespace
 
 // Returns 1 when it launched, 0 when the request is outside its form, negative on error.
-int try_gemm_wide(const GemmArgs& g, bool out_f32, hipStream_t stream) {
-  const bool res = g.res != nullptr;
-  if (out_f32 != res || (res && g.act != ACT_NONE)) return 0;
-  if (g.N % GW_T != 0 || g.K % GW_BK != 0 || g.K < 2 * GW_BK) return 0;
+int try_gemm_wide(const GemmArgs& g, hipStream_t stream) {
+  if (g.N % GW_T != 0 || g.K % GW_BK != 0 || g.K > (1 << 20) || g.M > 0x7fffffff - GW_T) return 0;
+  // long K (at 1024 the two forms are equal, 57 us at 65500 x 256) and rounds of tiles that fill the CUs: a last round
+  // of an eighth costs what it would full (24576 x 768 x 3072, 288 tiles: 163 us in the other form, 180 here)
   const int64_t tiles = cdiv(g.M, GW_T) * (g.N / GW_T);
-  if (tiles < 256 || tiles > 0x3fffffff || g.M > 0x7fffffff - GW_T || g.K > (1 << 20)) return 0;
+  if (g.K < 2048 || tiles > 0x3fffffff || tiles < 256 || tiles * 4 < cdiv(tiles, 256) * 256 * 3) return 0;
   if (g.M * g.ld_x * 2 > 0xffffffffll || g.N * g.ld_w * 2 > 0xffffffffll) return 0;
   WideArgs a = {};
   a.M = (int)g.M;
@@ -282,13 +271,7 @@ int try_gemm_wide(const GemmArgs& g, bool out_f32, hipStream_t stream) {
   a.ld_out = g.ld_out;
   a.nt = (int)(g.N / GW_T);
   a.tiles = (int)tiles;
-  const dim3 grid(256), block(256);
-  if (res)
-    hipLaunchKernelGGL((gemm_wide_kernel<ACT_NONE, true>), grid, block, 0, stream, a);
-  else if (g.act == ACT_GELU)
-    hipLaunchKernelGGL((gemm_wide_kernel<ACT_GELU, false>), grid, block, 0, stream, a);
-  else
-    hipLaunchKernelGGL((gemm_wide_kernel<ACT_NONE, false>), grid, block, 0, stream, a);
+  hipLaunchKernelGGL(gemm_wide_kernel, dim3(256), dim3(256), 0, stream, a);
   CORTEX_CHECK_LAUNCH("gemm_wide_kernel");
   return 1;
 }

@@ -28,3 +28,31 @@ def test_large_linear_column_parameters(M, N, K, act):
         want = torch.nn.functional.gelu(want)
     assert ((got.double() - want).norm() <= 2.0 ** -8 * want.norm())
     assert ((got.double() - want).abs().amax() <= 2.0 ** -8 * want.abs().amax() + 2.0 ** -8)
+
+
+@pytest.mark.parametrize("M,N,K", [(65536, 256, 2048), (65300, 256, 2112), (32769, 512, 2048), (21900, 768, 3072),
+                                   (98400, 256, 2048)])
+@pytest.mark.parametrize("res_rows", [0, 384])
+def test_wide_residual_linear(M, N, K, res_rows):
+    """The persistent 256 x 256 residual GEMM (long K, rounds of tiles that fill the CUs): partial last rows,
+    one to two rounds, an odd number of K stages, a broadcast residual and one updated in place; sampled
+    rows against 64 bits (K / 16 + 8 accumulations of 2^-24 of sum |a| |w|)."""
+    from cortex.kernels import ops
+
+    g = torch.Generator(DEV).manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
+    s = torch.rand(N, generator=g, device=DEV) + 0.5
+    b = torch.randn(N, generator=g, device=DEV)
+    rows = torch.cat([torch.randint(0, M, (500,), generator=g, device=DEV), torch.arange(M - 300, M, device=DEV)])
+    y = x[rows].double() @ w.double().t().contiguous() * s.double()
+    mag = x[rows].double().abs() @ w.double().abs().t().contiguous() * s.double() + 8
+    if res_rows:
+        res = torch.randn(res_rows, N, generator=g, device=DEV)
+        got = ops.norm_linear(x, weight=w, weight_scale=s, residual=res, res_rows=res_rows, out_dtype=torch.float32)
+        want = y + res[rows % res_rows].double()
+    else:
+        got = torch.randn(M, N, generator=g, device=DEV)
+        want = y + b.double() + got[rows].double()
+        ops.norm_linear(x, weight=w, weight_scale=s, bias=b, residual=got, out=got, out_dtype=torch.float32)
+    assert ((got[rows] - want).abs() <= (K / 16 + 8) * 2.0 ** -24 * mag).all()
