@@ -154,7 +154,7 @@ __device__ __forceinline__ void rowln_epilogue(const RowLnArgs& g, const ACC (&a
   // (lane sums, then xor-shuffles over the 4 lane groups), and the 8 equal-sized
   // parts combine as mean = avg(mean_w), M2 = sum(M2_w) + WN * sum((mean_w - mean)^2)
   // (Chan, Golub and LeVeque's pairwise update), as stable as two full passes.
-  float2* red = reinterpret_cast<float2*>(smem);  // [RL_WAVES][RL_BM]
+  float2* red = reinterpret_cast<float2*>(smem);  // [RL_WAVES][16 TM]
   constexpr float inv_wn = 1.0f / (float)WN;
   float mean[TM], rstd[TM];
   __syncthreads();  // every operand read of the LDS is done: it may be reused
@@ -178,7 +178,7 @@ __device__ __forceinline__ void rowln_epilogue(const RowLnArgs& g, const ACC (&a
       }
     m2 += __shfl_xor(m2, 16, 64);
     m2 += __shfl_xor(m2, 32, 64);
-    if (g4 == 0) red[cb * RL_BM + i * 16 + fr] = make_float2(mw, m2);
+    if (g4 == 0) red[cb * (16 * TM) + i * 16 + fr] = make_float2(mw, m2);
   }
   __syncthreads();
 #pragma unroll
@@ -187,7 +187,7 @@ __device__ __forceinline__ void rowln_epilogue(const RowLnArgs& g, const ACC (&a
     float msum = 0.0f;
 #pragma unroll
     for (int w = 0; w < RL_WAVES; ++w) {
-      part[w] = red[w * RL_BM + i * 16 + fr];
+      part[w] = red[w * (16 * TM) + i * 16 + fr];
       msum += part[w].x;
     }
     const float mu = msum * (1.0f / (float)RL_WAVES);
@@ -415,17 +415,18 @@ __global__ __launch_bounds__(RL_THREADS) void gemm_rowln_kernel(RowLnArgs g) {
 // rows, half lines, which measured slower than the LDS ring.)  The 32 A rows, which every
 // wavefront reads, move into LDS once before the loop (all of K: 32 * K * 2 bytes, the ring's
 // swizzled layout, one 64-deep K step per 4 KiB).  Same fragments and the same accumulation
-// order as the ring form, so the results are bit-identical to it.
+// order as the ring form, so the results are bit-identical to it.  BM: 32 rows, or 64 (twice the accumulators
+// and residual registers, half the weight reads per row).
 constexpr int RL_DW_AHEAD = 2;  // 2: forward 0.6945-0.6968 ms; 3: 0.6970-0.6990; 4: 0.6961-0.6986
 
-template <int BN, int NK, bool Q8>
+template <int BN, int NK, bool Q8, int BM = RL_BM>
 __global__ __launch_bounds__(RL_THREADS) void gemm_rowln_dw_kernel(RowLnArgs g) {
   using OP = Operand<bf16>;
   typedef typename OP::frag frag;
-  constexpr int WN = BN / RL_WAVES, TM = RL_BM / 16, TN = WN / 16, WD = RL_DW_AHEAD;
-  constexpr int A_STAGE = RL_BM * 128;                   // 32 rows x 64 K of bf16
+  constexpr int WN = BN / RL_WAVES, TM = BM / 16, TN = WN / 16, WD = RL_DW_AHEAD;
+  constexpr int A_STAGE = BM * 128;                      // the rows x 64 K of bf16
   constexpr int AB = NK * (A_STAGE / 1024) / RL_WAVES;   // 1 KiB A transfers per wavefront
-  constexpr int RED = RL_WAVES * RL_BM * 8;              // the epilogue's statistics exchange
+  constexpr int RED = RL_WAVES * BM * 8;                 // the epilogue's statistics exchange
   constexpr int LDS = NK * A_STAGE > RED ? NK * A_STAGE : RED;
   constexpr int RV = TM * TN, WOPS = TN * 2;             // residual loads; W loads per K step
   static_assert(NK * (A_STAGE / 1024) % RL_WAVES == 0 && NK >= WD && TN >= 1, "shape");
@@ -435,20 +436,20 @@ __global__ __launch_bounds__(RL_THREADS) void gemm_rowln_dw_kernel(RowLnArgs g) 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int fr = lane & 15, g4 = lane >> 4;
   const int M = (int)g.M;
-  const int m0 = blockIdx.x * RL_BM;
+  const int m0 = blockIdx.x * BM;
   // column block of this wavefront, rotated by workgroup: at any moment the workgroups of an
   // XCD stream 8 different weight blocks rather than all the same 4 KiB per wavefront index
   // (out-projection at B = 32: 16.34-16.41 -> 16.13-16.20 us, same box)
   const int cb = (wid + (int)blockIdx.x) & (RL_WAVES - 1);
   const int wcol = cb * WN;
 
-  // A: the 1 KiB block q = wid * AB + i holds rows 8 (q % 4) .. +7 of K step q / 4 (lane i of a
+  // A: the 1 KiB block q = wid * AB + i holds rows 8 (q % (BM / 8)) .. +7 of K step q / (BM / 8) (lane i of a
   // transfer: row i / 8, stored chunk i % 8 = logical chunk (i % 8) ^ rl_swz(row))
   const bf16* A = reinterpret_cast<const bf16*>(g.x);
 #pragma unroll
   for (int i = 0; i < AB; ++i) {
-    const int q = wid * AB + i, r = (q & 3) * 8 + (lane >> 3);
-    const bf16* src = A + (int64_t)min(m0 + r, M - 1) * g.ld_x + (q >> 2) * 64 + ((lane & 7) ^ rl_swz(r)) * 8;
+    const int q = wid * AB + i, r = q % (BM / 8) * 8 + (lane >> 3);
+    const bf16* src = A + (int64_t)min(m0 + r, M - 1) * g.ld_x + q / (BM / 8) * 64 + ((lane & 7) ^ rl_swz(r)) * 8;
     __builtin_amdgcn_global_load_lds(static_cast<const void*>(src), static_cast<void*>(smem + q * 1024), 16, 0, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(RL_THREADS) void gemm_rowln_dw_kernel(RowLnArgs g) 
     a_sw[t] = rl_swz(r);
   }
   rl_wait_vm<RV + WD * WOPS>();  // this wave's A transfers landed (the W and residual loads came after)
-  __builtin_amdgcn_s_barrier();  // every wave's: all 32 A rows in LDS
+  __builtin_amdgcn_s_barrier();  // every wave's: all A rows in LDS
 #pragma unroll
   for (int kt = 0; kt < NK; ++kt) {
     const unsigned char* as = smem + kt * A_STAGE;
@@ -554,9 +555,14 @@ int residual_ln(const char* who, int64_t M, int64_t N, int64_t K, const void* x,
               gamma, beta,  eps,   xn,  ld_xn, q8 ? 1.0f / xq_scale : 0.0f, a_scale};
   const dim3 grid((unsigned)cdiv(M, (int64_t)RL_BM));
   if (frag) {  // bf16 rows x the fragment-order weight: the direct-weight form
+    // 64 rows a workgroup past one workgroup of 32 per CU: the weight is streamed once per workgroup, and 32-row
+    // ones would come in rounds (N = K = 512: 8704 rows 28.5 -> 21.4 us, 16384 32.8 -> 27.2, 32768 60.5 -> 53.8,
+    // 65536 129.3 -> 128.6; 256: 8448 12.9 -> 10.3, 32768 25.2 -> 25.3)
+    const bool tall = M > 256 * RL_BM;
 #define RL_DW(BN_, NK_)                                                                                           \
   do {                                                                                                            \
     if (q8) hipLaunchKernelGGL((gemm_rowln_dw_kernel<BN_, NK_, true>), grid, dim3(RL_THREADS), 0, stream, a);   \
+    else if (tall) hipLaunchKernelGGL((gemm_rowln_dw_kernel<BN_, NK_, false, 64>), dim3((unsigned)cdiv(M, (int64_t)64)), dim3(RL_THREADS), 0, stream, a); \
     else hipLaunchKernelGGL((gemm_rowln_dw_kernel<BN_, NK_, false>), grid, dim3(RL_THREADS), 0, stream, a);     \
   } while (0)
     if (N == 512 && K == 512) RL_DW(512, 8);

@@ -56,3 +56,24 @@ def test_wide_residual_linear(M, N, K, res_rows):
         want = y + b.double() + got[rows].double()
         ops.norm_linear(x, weight=w, weight_scale=s, bias=b, residual=got, out=got, out_dtype=torch.float32)
     assert ((got[rows] - want).abs() <= (K / 16 + 8) * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("M", [8192, 8193, 8250, 8256, 16385, 20001])
+@pytest.mark.parametrize("N,K", [(256, 256), (256, 512), (512, 256), (512, 512)])
+@pytest.mark.parametrize("res_rows", [0, 256])
+def test_tall_residual_layer_norm_equals_ring(M, N, K, res_rows):
+    """The 64-row direct-weight form (past 8192 rows) gives the plain-row kernel's bits, at partial last
+    workgroups, with a broadcast residual and in place."""
+    from cortex.kernels import ops
+
+    g = torch.Generator(DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=DEV) * 0.05).bfloat16()
+    s, b, gm, bt = (torch.rand(N, generator=g, device=DEV) + 0.5 for _ in range(4))
+    res = torch.randn(res_rows or M, N, generator=g, device=DEV)
+    ln = (gm, bt, 1e-5)
+    want = ops.linear_residual_ln(x, w, s, b, residual=res, ln=ln, res_rows=res_rows)
+    out = None if res_rows else res.clone()
+    got = ops.linear_residual_ln(x, ops.frag_weight(w), s, b, residual=res if out is None else out, ln=ln,
+                                 res_rows=res_rows, out=out, frag=True)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
