@@ -989,16 +989,26 @@ int launch_res_dw_impl(const GemmArgs& g, hipStream_t stream) {
   return OK;
 }
 
-// Tile by shape: 256-row tiles halve the operand traffic per MFMA, so take the widest tile
-// that still fills (nearly) every CU once, else 128 x 128 (two workgroups per CU).
+// Tile by shape.  A launch takes whole rounds: one tile of 256 x 256 or 256 x 192 per CU and round (a round with a few
+// tiles costs what a full one does), 128 x 128 ones two to a CU.  In rounds of 256 x 256 tiles a round of 256 x 192
+// takes 0.73 (K = 512) to 0.84, one 128 x 128 tile per CU 0.45 .. 0.57, two 0.69 .. 0.82, more 0.40 + 0.27 per CU's worth;
+// the least of the three (past three rounds the persistent 256 x 256 tiles lead again).  Measured, us (fill a CU
+// nearly once, else 128 x 128 -> this rule): 3072 x 3072 x 768 GELU 29.0 -> 21.6, 4096 x 2304 x 768 26.3 -> 19.8, 9216 x
+// 2304 x 768 51.1 -> 42.0, 6144 x 1536 x 512 19.3 -> 14.5, 12288 x 1536 x 512 34.7 -> 28.8, 9216 x 2048 x 512 GELU 38.9 -> 32.5,
+// 12288 x 768 x 256 13.3 -> 9.9, 4608 x 2048 x 512 GELU 22.2 -> 19.6.
 enum TileChoice { T128 = 0, T256 = 4, T192 = 6, T128_K2 = 7 };
 TileChoice wide_tile(const GemmArgs& g, bool allow192) {
-  const int64_t t256 = cdiv(g.M, 256) * cdiv(g.N, 256), t192 = cdiv(g.M, 256) * cdiv(g.N, 192);
   const int ncu = cu_count();
-  if (g.N % 256 == 0 && t256 >= ncu * 15 / 16) return T256;
-  if (allow192 && g.N % 192 == 0 && t192 >= ncu * 15 / 16 && t192 <= ncu) return T192;
-  if (t256 >= ncu * 3 / 4) return T256;
-  return T128;
+  const int64_t t256 = cdiv(g.M, 256) * cdiv(g.N, 256), t192 = cdiv(g.M, 256) * cdiv(g.N, 192);
+  const int64_t t128 = cdiv(g.M, 128) * cdiv(g.N, 128);
+  // time in rounds of 256 x 256 tiles: whole rounds of one large tile per CU; 128 x 128 ones two to a CU, which past
+  // the first round follow one another without one
+  const double c256 = (double)cdiv(t256, ncu);
+  const int64_t r192 = cdiv(t192, ncu);
+  const double c192 = allow192 && g.N % 192 == 0 && r192 <= 3 ? 0.82 * r192 : 1e30;
+  const double c128 = t128 <= ncu ? 0.48 : t128 <= 2 * ncu ? 0.76 : 0.40 + 0.27 * t128 / ncu;
+  if (c128 < c256 && c128 < c192) return T128;
+  return c192 < c256 ? T192 : T256;
 }
 
 template <int ACT, bool RES, class TOUT, class TW = bf16>

@@ -77,3 +77,34 @@ def test_tall_residual_layer_norm_equals_ring(M, N, K, res_rows):
     got = ops.linear_residual_ln(x, ops.frag_weight(w), s, b, residual=res if out is None else out, ln=ln,
                                  res_rows=res_rows, out=out, frag=True)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("M,N", [(3069, 2304), (4093, 2304), (6141, 2304), (7679, 2304), (9213, 2304), (4605, 2048),
+                                 (12285, 768), (12285, 1536), (9213, 2048), (16381, 2304)])
+@pytest.mark.parametrize("form", ["image", "int8", "rms"])
+def test_tile_rule(M, N, form):
+    """Row counts on every side of the tile rule (128 x 128, 256 x 192 and 256 x 256 tiles in one to three
+    rounds), partial last tiles: sampled and last rows against 64 bits, 2^-8."""
+    from cortex.kernels import ops
+    from cortex.kernels.fused_rmsnorm import norm_linear_int8
+
+    K = 128
+    g = torch.Generator(DEV).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    q, s = ops.quantize_int8(torch.randn(N, K, generator=g, device=DEV) * 0.05)
+    wd = q.double() * s.double()[:, None]
+    rows = torch.cat([torch.randint(0, M, (400,), generator=g, device=DEV), torch.arange(M - 260, M, device=DEV)])
+    a = x[rows].double()
+    if form == "rms":
+        got = norm_linear_int8(x, q, s, gamma=torch.ones(K, device=DEV))
+        a = a / (a.square().mean(1, keepdim=True) + 1e-6).sqrt()
+    elif form == "int8":
+        got = ops.norm_linear(x, weight_int8=q, weight_scale=s, act="gelu", out_dtype=torch.bfloat16)
+    else:
+        got = ops.norm_linear(x, weight=ops.convert(q, torch.bfloat16), weight_scale=s, act="gelu",
+                              out_dtype=torch.bfloat16)
+    want = a @ wd.t().contiguous()
+    if form != "rms":
+        want = torch.nn.functional.gelu(want)
+    err = (got[rows].double() - want).abs()
+    assert (err.norm() <= 2.0 ** -8 * want.norm()) and (err.amax() <= 2.0 ** -7 * want.abs().amax())
