@@ -767,7 +767,7 @@ def _plain_bf16_linear(x, weight, weight_scale, bias, act, residual, res_rows, o
     questions that contiguous operands answer left out (half of a block's time on the host)."""
     dev = nat.require_gpu(x, weight, weight_scale, bias, residual, out, what="norm_linear")
     N, K = weight.shape
-    M = x.numel() // K if K else 0
+    M = x.numel() // K
     if out is None:
         out = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=dev)
     elif out.numel() != M * N:
@@ -802,7 +802,8 @@ def norm_linear(x: torch.Tensor, *, weight: torch.Tensor | None = None, weight_i
     """
     if (norm is None and weight is not None and weight.dtype is torch.bfloat16 and x.dtype is torch.bfloat16
             and compute_dtype is torch.bfloat16 and w_layout == "nk" and weight_int8 is None
-            and weight.dim() == 2 and x.shape[-1] == weight.shape[1] and x.is_contiguous() and weight.is_contiguous()
+            and weight.dim() == 2 and x.shape[-1] == weight.shape[1] > 0 and x.is_contiguous() and weight.is_contiguous()
+            and (residual is None or residual.shape[-1] == weight.shape[0])
             and all(t is None or t.is_contiguous() for t in (weight_scale, residual, out))):
         return _plain_bf16_linear(x, weight, weight_scale, bias, act, residual, res_rows, out_dtype or x.dtype, out)
     w = weight if weight is not None else weight_int8

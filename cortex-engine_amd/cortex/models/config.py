@@ -3,7 +3,7 @@
 Same fields, validation and the three reference sizes.  ``dtype`` -- declared but
 never read by the reference -- selects the MFMA input dtype of the HIP forward:
 ``"bfloat16"`` (default; bf16 operands, fp32 accumulation, fp32 residual stream)
-or ``"float32"`` (fp32 operands on fp32 MFMA).
+or ``"float32"`` (fp32 operands, as exact sums of bf16 parts on the MFMA).
 """
 
 from __future__ import annotations

@@ -280,7 +280,8 @@ class CortexModel(nn.Module):
                       ops.heads_view(kv, 1, E, H, D, D), kv_offsets=offsets, out=o, batch=B)
         first = enc.self_attn_blocks[0] if len(enc.self_attn_blocks) else None
         few = ops.small_linear_ok(B * L, D, D) and small_ok(xa.out_proj, o_buf, compute)
-        if not few and first is not None and residual_ln_ok(xa.out_proj, first.norm_attn, first.qkv_proj, enc.latents, compute):
+        if not few and first is not None and residual_ln_ok(xa.out_proj, first.norm_attn, first.qkv_proj, enc.latents,
+                                                            compute):
             # latents + out_proj(attn) and the first block's norm_attn in one launch
             return linear_residual_ln(xa.out_proj, o_buf, enc.latents, first.norm_attn, res_rows=L,
                                       out=torch.empty(B * L, D, dtype=torch.float32, device=kv.device))

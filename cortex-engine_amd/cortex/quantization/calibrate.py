@@ -134,7 +134,7 @@ class QuantizedLinear(nn.Module):
 
     ``forward`` runs the HIP INT8 GEMM: int8 weights widened exactly inside the
     kernel, fp32 accumulation, ``* weight_scale[n] (+ bias[n])`` in the epilogue;
-    output in ``x.dtype`` (bf16 inputs use bf16 MFMA, fp32 inputs fp32 MFMA).
+    output in ``x.dtype`` (bf16 inputs use bf16 MFMA, fp32 inputs their exact bf16 parts).
     """
 
     in_features: int

@@ -13,8 +13,9 @@
 // one piece.  From plain rows it is 64 bytes of 16 rows, which a CU took in at 21 bytes a cycle whatever the number of
 // wavefronts or the MFMA shape (256 x 512 x 2048: 9.4 us, 4.3 this way); the MLP's hidden rows are written and read
 // in that order too.  (int8 rows, for weights that stay int8 in memory, are widened
-// before their MFMAs: the same values in the same order, the same results.)  The price is operand traffic (every tile reads 32 rows of each operand, 32 MB of L2 reads at
-// 256 x 2048 x 512), so larger row counts keep the larger tiles (the rule: small_linear_ok in ops.py).
+// before their MFMAs: the same values in the same order, the same results.)  The price is operand traffic (every
+// tile reads 32 rows of each operand, 32 MB of L2 reads at 256 x 2048 x 512), so larger row counts keep the larger
+// tiles (the rule: small_linear_ok in ops.py).
 //
 // With LayerNorm (K up to 1024) the wavefront holds its K part of the 32 fp32 rows in registers: two
 // exchanges of partial sums give mean and variance (two passes over registers), and no row kernel runs
@@ -297,7 +298,8 @@ extern "C" int cortex_linear_small(int64_t M, int64_t N, int64_t K, int x_dtype,
                        (!residual || ld_res >= N),
                    "cortex_linear_small: a row stride is smaller than its row");
   auto a16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  CORTEX_CHECK_ARG(a16(x) && (x_dtype == DT_BF16_FRAG || ld_x % (ln ? 4 : 8) == 0) && (w_dtype == DT_I8 ? ((uintptr_t)w & 7) == 0 && ld_w % 8 == 0 : a16(w)) && a16(gamma) &&
+  CORTEX_CHECK_ARG(a16(x) && (x_dtype == DT_BF16_FRAG || ld_x % (ln ? 4 : 8) == 0) &&
+                       (w_dtype == DT_I8 ? ((uintptr_t)w & 7) == 0 && ld_w % 8 == 0 : a16(w)) && a16(gamma) &&
                        a16(beta) && (out_dtype != DT_BF16_FRAG || a16(out)),
                    "cortex_linear_small: operands must be 16-byte aligned rows");
   CORTEX_CHECK_ARG(M <= (1 << 20) && N <= (1 << 20) && res_rows <= (1 << 20), "cortex_linear_small: shape too large");
