@@ -778,7 +778,7 @@ def weights_and_modes(model, dev, inputs, reference: torch.Tensor) -> dict:
     sec_f, out_f = _time_captured(f32, dev, inputs, reps=20)
     res["fp32_compute"] = {"ms_per_forward": round(sec_f * 1e3, 4), "samples_per_s": round(B_MAIN / sec_f, 1),
                            "max_abs_diff_vs_default": float((out_f - reference).abs().max()),
-                           "note": "fp32 activations and fp32 MFMA with the INT8 weights dequantised in the "
+                           "note": "fp32 activations (exact bf16 parts on the MFMA, fp32 sums) with the INT8 weights dequantised in the "
                                    "kernel: the reference QuantizedLinear arithmetic (1e-5 parity bar)"}
     del f32
     torch.cuda.empty_cache()
