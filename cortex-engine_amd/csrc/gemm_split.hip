@@ -471,7 +471,7 @@ int launch_split(SplitArgs g, hipStream_t stream) {
   return OK;
 }
 
-constexpr int64_t SP_A_MAX = 256ll << 20;  // planes of the rows, at most, in the workspace asked for
+constexpr int64_t SP_A_MAX = 256ll << 20;  // planes of the rows, at most, in the workspace asked for (128 have to fit)
 constexpr int64_t SP_W_MAX = 256ll << 20;  // planes of the weight; a larger one is not taken
 
 int64_t w_plane_bytes(int64_t N, int64_t K, int w_dtype) {
@@ -492,8 +492,9 @@ int64_t cortex_norm_linear_split_workspace_bytes(int64_t M, int64_t N, int64_t K
   if (M < 1 || N < 1 || K < 1 || (w_dtype != DT_I8 && w_dtype != DT_F32)) return 0;
   if (N > (1ll << 31) || K > (1ll << 24) || w_plane_bytes(N, K, w_dtype) > SP_W_MAX) return 0;
   const int64_t per = chunk_bytes(K);
+  if (per > SP_A_MAX) return 0;
   int64_t chunks = cdiv(M, 128);
-  if (chunks * per > SP_A_MAX) chunks = SP_A_MAX / per > 0 ? SP_A_MAX / per : 1;
+  if (chunks * per > SP_A_MAX) chunks = SP_A_MAX / per;
   return w_plane_bytes(N, K, w_dtype) + chunks * per;
 }
 

@@ -275,7 +275,7 @@ int cortex_linear_small(int64_t M, int64_t N, int64_t K, int x_dtype, const void
  * gamma_dtype 0, 1 or 2); w_scale, bias optional fp32; act, residual and res_rows as
  * cortex_norm_linear; out may be residual.  The workspace (16-byte aligned) holds the parts of the
  * weight and of as many rows as fit: cortex_norm_linear_split_workspace_bytes gives the size that
- * takes up to 256 MiB of rows at once (0: a weight too large for this form); a smaller one, down to
+ * takes up to 256 MiB of rows at once (0: a weight, or 128 rows, too large for this form); a smaller one, down to
  * 128 rows, only costs more launches. */
 int64_t cortex_norm_linear_split_workspace_bytes(int64_t M, int64_t N, int64_t K, int w_dtype);
 int cortex_norm_linear_split(int64_t M, int64_t N, int64_t K, const float* x, int64_t ld_x, int norm,
