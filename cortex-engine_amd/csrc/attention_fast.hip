@@ -9,7 +9,9 @@
 // then runs over that list exactly as over dense tiles (no load of the tile loop has a register
 // destination), and a tile that is not all ones masks its scores from its word.  Up to AF_KM_TILES
 // tiles (5 KiB of LDS beside the ring's 64: two workgroups still share a CU).  Against the general
-// kernel, B 32, H 8, 256 x 512 keys padded to 128 .. 512: 71.5 -> 17.9 us.
+// kernel, B 32, H 8, 256 x 512 keys padded to 128 .. 512: 71.5 -> 18.5 .. 20.0 us, at its precision: the
+// lagging reference max and the sum of rounded probabilities that dense keys use would take 16.7 .. 17.7
+// and be 5 % further from 64 bits (2.260e-3 against 2.155e-3 on N(0, 1) queries and keys).
 //
 // Workgroup: 8 wavefronts x 16 or 32 queries of one (sample, head).  Keys are taken in
 // chunks of up to 4 tiles of 64: every load of a chunk is issued at once (one
@@ -211,11 +213,15 @@ void attention_fast_kernel(AttnArgs a) {
       v_off[c][t] = r * 128 + (((d >> 3) ^ vswz(r)) << 4) + ((d >> 2) & 1) * 8;
     }
 
-  float m_run[QG];
+  // Per-key masks keep the general kernel's precision: the reference max is the running max (the
+  // largest probability is 1, exact in bf16) and the sum takes the probabilities before their rounding.
+  constexpr float RESCALE = KM ? 0.0f : AF_RESCALE;
+  float m_run[QG], l_sum[QG];  // l_sum: this lane group's keys (KM)
   f32x4 o_acc[QG][4], l_acc[QG];
 #pragma unroll
   for (int qg = 0; qg < QG; ++qg) {
     m_run[qg] = -INFINITY;
+    l_sum[qg] = 0.0f;
     l_acc[qg] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int t = 0; t < 4; ++t) o_acc[qg][t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
@@ -326,14 +332,14 @@ void attention_fast_kernel(AttnArgs a) {
     for (int qg = 0; qg < QG; ++qg) {
       if (!okq[qg]) continue;
       // Lane-local max first: the reference max only has to move (and the lane groups
-      // only have to agree on a new one) when some score exceeds it by AF_RESCALE.
+      // only have to agree on a new one) when some score exceeds it by RESCALE.
       float mx = s[qg][0][0];
 #pragma unroll
       for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[qg][st][i]);
       // wave-uniform, rare after the group's first tile (m_run = -inf always enters)
-      if (__any(mx * sl > m_run[qg] + AF_RESCALE)) {
+      if (__any(mx * sl > m_run[qg] + RESCALE)) {
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         const float m_tile = mx * sl;  // finite: every tile holds at least one valid key
@@ -344,6 +350,7 @@ void attention_fast_kernel(AttnArgs a) {
           const float alpha = __builtin_amdgcn_exp2f(m_run[qg] - m_new);
           m_run[qg] = m_new;
           l_acc[qg] *= alpha;
+          l_sum[qg] *= alpha;
 #pragma unroll
           for (int t = 0; t < 4; ++t) o_acc[qg][t] *= alpha;
         }
@@ -352,15 +359,18 @@ void attention_fast_kernel(AttnArgs a) {
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          pf[qg][c][i] = (bf16)__builtin_amdgcn_exp2f(fmaf(s[qg][2 * c][i], sl, -m_run[qg]));  // -inf -> 0
-          pf[qg][c][4 + i] = (bf16)__builtin_amdgcn_exp2f(fmaf(s[qg][2 * c + 1][i], sl, -m_run[qg]));
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[qg][2 * c][i], sl, -m_run[qg]));  // -inf -> 0
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(s[qg][2 * c + 1][i], sl, -m_run[qg]));
+          if constexpr (KM) l_sum[qg] += p0 + p1;
+          pf[qg][c][i] = (bf16)p0;
+          pf[qg][c][4 + i] = (bf16)p1;
         }
     }
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
 #pragma unroll
       for (int qg = 0; qg < QG; ++qg)
-        if (okq[qg]) l_acc[qg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[qg][c], l_acc[qg], 0, 0, 0);
+        if (!KM && okq[qg]) l_acc[qg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[qg][c], l_acc[qg], 0, 0, 0);
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const uint2 v0 = lds_read_tr16(vs_ + v_off[c][t]), v1 = lds_read_tr16(vs_ + v_off[c][t] + 4 * 128);
@@ -464,7 +474,11 @@ void attention_fast_kernel(AttnArgs a) {
 
 #pragma unroll
   for (int qg = 0; qg < QG; ++qg) {
-    const float l = l_acc[qg][0];
+    float l = l_acc[qg][0];
+    if constexpr (KM) {
+      l = l_sum[qg] + __shfl_xor(l_sum[qg], 16, 64);
+      l += __shfl_xor(l, 32, 64);
+    }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     const int64_t q = q0 + 16 * qg + fr;
     if (q < a.Lq) {
