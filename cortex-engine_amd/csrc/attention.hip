@@ -209,14 +209,17 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_kernel(AttnArgs a) {
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
     const float m_new = fmaxf(m_run, tmax);
-    if (m_new != -INFINITY) {
-      const float alpha = exp2f(m_run - m_new);  // m_run = -inf -> 0
+    // the whole wavefront or none of it: an MFMA takes every lane's operands, also those of a lane
+    // whose query has no allowed key so far (all its probabilities are exp2(-inf) = 0)
+    if (__any(m_new != -INFINITY)) {
+      const float ref = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = exp2f(m_run - ref);  // m_run = -inf -> 0
       float psum = 0.0f;
 #pragma unroll
       for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float p = exp2f(s[st][i] - m_new);  // masked -> 0
+          const float p = exp2f(s[st][i] - ref);  // masked -> 0
           s[st][i] = p;
           psum += p;
         }

@@ -77,6 +77,29 @@ def test_all_masked_rows_are_zero_and_partial_tiles():
     assert (out[:, :, 16:32].cpu() == 0).all()
 
 
+@pytest.mark.parametrize("L,E,Dh,bl,be", [(40, 70, 32, 1, 1), (40, 70, 64, 1, 1), (72, 200, 64, 24, 128), (33, 130, 128, 5, 64),
+                                          (200, 300, 64, 1, 7)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tiles_that_split_a_wavefront(L, E, Dh, bl, be, dtype):
+    """Mask tiles whose edges fall inside 16 queries (and rows past the last query): the queries of one
+    wavefront start on different key tiles, some on none."""
+    from cortex.kernels.sparse_xattn import sparse_cross_attention
+
+    q, k, v = _qkv(2, 3, L, E, Dh, dtype, seed=L + E)
+    g = torch.Generator().manual_seed(bl)
+    mask = torch.rand(math.ceil(L / bl), math.ceil(E / be), generator=g) < 0.5
+    mask[0] = False
+    mask[1, : (mask.shape[1] + 1) // 2] = False
+    kpm = torch.rand(2, E, generator=g) < 0.8
+    for pad in (None, kpm):
+        out = sparse_cross_attention(q.to(DEV), k.to(DEV), v.to(DEV), mask, BLOCK_L=bl, BLOCK_E=be,
+                                     key_padding_mask=pad.to(DEV) if pad is not None else None)
+        allowed = mask.repeat_interleave(bl, 0)[:L].repeat_interleave(be, 1)[:, :E]
+        allowed = allowed if pad is None else allowed & pad[:, None, None, :]
+        ref = O.attention_bruteforce_f64(q.float(), k.float(), v.float(), allowed=allowed.expand(2, 3, L, E).numpy())
+        _close(out.float().cpu().numpy(), ref, 1e-5 if dtype == torch.float32 else 1e-2)
+
+
 def test_config1_ragged_lengths_bf16():
     """Config 1: B=32, L=256, E_pad=512, Dh=64, bf16, true lengths U[128,512], N(0,1)/sqrt(64)."""
     from cortex.kernels.sparse_xattn import sparse_cross_attention
