@@ -318,9 +318,10 @@ def qkv_attention(xn: torch.Tensor, weight: torch.Tensor, weight_scale, bias, ba
 
 
 def frag_weight(weight: torch.Tensor) -> torch.Tensor:
-    """The (N, K) weight (int8, bf16 or fp32) as bf16 in MFMA fragment order
-    (``cortex_frag_weight``), shape (N, K) but not row-major: only ``linear_residual_ln(...,
-    frag=True)`` reads it.  Values exactly those of ``convert(weight, torch.bfloat16)``."""
+    """The (N, K) weight (int8, bf16, fp16 or fp32) as bf16 in MFMA fragment order
+    (``cortex_frag_weight``), shape (N, K) but not row-major: ``linear_residual_ln(..., frag=True)``,
+    ``linear_residual_frag`` and ``linear_small`` read it.  Values exactly those of
+    ``convert(weight, torch.bfloat16)``, from every dtype that takes."""
     dev = nat.require_gpu(weight, what="frag_weight")
     w2 = _row_major_2d(weight)
     N, K = w2.shape

@@ -643,8 +643,8 @@ int cortex_frag_weight(int64_t N, int64_t K, const void* w, int w_dtype, int64_t
   if (N == 0 || K == 0) return OK;
   CORTEX_CHECK_ARG(N % 16 == 0 && K % 32 == 0, "%s: N must be a multiple of 16 and K of 32", who);
   CORTEX_CHECK_ARG(w && out && ld_w >= K, "%s: null pointer or short rows", who);
-  CORTEX_CHECK_ARG(w_dtype == DT_I8 || w_dtype == DT_BF16 || w_dtype == DT_F32, "%s: weight must be int8, bf16 or fp32",
-                   who);
+  CORTEX_CHECK_ARG(w_dtype == DT_I8 || w_dtype == DT_BF16 || w_dtype == DT_F32 || w_dtype == DT_F16,
+                   "%s: weight must be int8, bf16, fp16 or fp32", who);
   CORTEX_CHECK_ARG(((uintptr_t)out & 15) == 0, "%s: output must be 16-byte aligned", who);
   const int64_t chunks = N * K / 8;
   CORTEX_CHECK_ARG(cdiv(chunks, (int64_t)256) <= 0x7fffffffLL, "%s: too large", who);
@@ -654,6 +654,9 @@ int cortex_frag_weight(int64_t N, int64_t K, const void* w, int w_dtype, int64_t
                        (bf16*)out);
   else if (w_dtype == DT_BF16)
     hipLaunchKernelGGL(frag_weight_kernel<bf16>, grid, dim3(256), 0, stream, (const bf16*)w, ld_w, K, chunks,
+                       (bf16*)out);
+  else if (w_dtype == DT_F16)
+    hipLaunchKernelGGL(frag_weight_kernel<f16>, grid, dim3(256), 0, stream, (const f16*)w, ld_w, K, chunks,
                        (bf16*)out);
   else
     hipLaunchKernelGGL(frag_weight_kernel<float>, grid, dim3(256), 0, stream, (const float*)w, ld_w, K, chunks,

@@ -174,13 +174,13 @@ int cortex_transpose_bf16(int64_t R, int64_t C, const void* in, int64_t ld_in, v
  * norm 2 and gamma = NULL then applies the per-row 1 / rms to the fp32 accumulator. */
 int cortex_fold_gain(int64_t N, int64_t K, const void* w, int w_dtype, int kn, int64_t ld_w, const void* gamma,
                      int gamma_dtype, void* out, int64_t ld_out, hipStream_t stream);
-/* An (N, K) weight (int8, bf16 or fp32 rows: w_dtype 3 / 1 / 0) as bf16 in MFMA fragment
+/* An (N, K) weight (int8, bf16, fp16 or fp32 rows: w_dtype 3 / 1 / 2 / 0) as bf16 in MFMA fragment
  * order, the layout of weight code 7: 1 KiB block (n16, k32) = n16 * (K / 32) + k32 holds rows
  * 16 n16 .. +15 and K 32 k32 .. +31 as 64 lanes x 8 values, lane l = row 16 n16 + l % 16,
  * K 32 k32 + 8 (l / 16) .. +7.  Values as cortex_convert writes them (int8 exact).  Built once
  * per weight, like the bf16 image of QuantizedLinear's dequantised weight (calibrate.py:
- * 225-228), for cortex_linear_residual_ln.  N % 16 == 0, K % 32 == 0, out (N * K bf16)
- * 16-byte aligned. */
+ * 225-228), for cortex_linear_residual_ln, cortex_norm_linear's residual form and
+ * cortex_linear_small.  N % 16 == 0, K % 32 == 0, out (N * K bf16) 16-byte aligned. */
 int cortex_frag_weight(int64_t N, int64_t K, const void* w, int w_dtype, int64_t ld_w, void* out,
                        hipStream_t stream);
 

@@ -94,3 +94,29 @@ def test_block_around_the_few_row_rule(model, batch):
         got, want = blk(x), ref(x)
     # (bf16 operands, and a float weight rounded to bf16: a few bf16 steps of the branches' size)
     assert ((got - want).norm() <= 1e-2 * (want - x).norm())
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+def test_float16_weights_at_few_rows(batch):
+    """float16 nn.Linear weights run as their bf16 rounding, which fp32 weights of the same values have too."""
+    from cortex.kernels import ops
+    from cortex.models import config
+    from cortex.models.perceiver import CrossAttentionBlock, SelfAttentionBlock
+
+    cfg = config.CORTEX_S
+    torch.manual_seed(1)
+    for cls in (SelfAttentionBlock, CrossAttentionBlock):
+        blk, ref = cls(cfg).to(DEV).eval(), cls(cfg).to(DEV).eval()
+        for a, b in zip(blk.modules(), ref.modules()):
+            if isinstance(a, torch.nn.Linear):
+                a.weight.data = a.weight.data.half()
+                b.weight.data = a.weight.data.float()
+            elif isinstance(a, torch.nn.LayerNorm):
+                b.load_state_dict(a.state_dict())
+        args = [torch.randn(batch, cfg.num_latents, cfg.latent_dim, device=DEV)]
+        if cls is CrossAttentionBlock:
+            args.append(torch.randn(batch, 70, cfg.hidden_dim, device=DEV))
+        with torch.no_grad():
+            assert torch.equal(blk(*args), ref(*args))
+    w = torch.randn(64, 96, device=DEV).half()
+    assert torch.equal(ops.frag_weight(w), ops.frag_weight(w.bfloat16()))
