@@ -750,6 +750,10 @@ def linear_small(x: torch.Tensor, weight: torch.Tensor, weight_scale=None, bias=
     N = weight.shape[0]
     if weight.shape[1] != K:
         raise ValueError(f"inner dims differ: x has K={K}, weight has K={weight.shape[1]}")
+    if not x_frag:  # (expanded or overlapping rows are copied)
+        x = _row_major_2d(x)
+    if residual is not None:
+        residual = _row_major_2d(residual)
     if out is None:
         out = torch.empty((ceil_div(M, 16) * 16 if out_frag else M, N), dtype=out_dtype, device=dev)
     g, b, eps = ln if ln is not None else (None, None, 0.0)

@@ -369,12 +369,13 @@ def linear_residual_ln(lin: nn.Module, a: torch.Tensor, residual: torch.Tensor, 
 
 def small_ok(lin: nn.Module, x: torch.Tensor, compute: torch.dtype, norm: nn.LayerNorm | None = None) -> bool:
     """Whether ``lin`` (after ``norm``) can run as ``ops.linear_small`` on rows of ``x``, sizes aside: bf16
-    compute, no calibration hooks, fp32 parameters."""
+    compute, no calibration hooks, an fp32 bias, and an int8 weight of aligned rows with a contiguous scale."""
     if compute != torch.bfloat16 or lin._forward_pre_hooks or (norm is not None and norm._forward_pre_hooks):
         return False
-    if hasattr(lin, "weight_int8") and INT8_WEIGHTS != "image":
+    if hasattr(lin, "weight_int8"):
         q = lin.weight_int8
-        if q.dim() != 2 or q.stride(1) != 1 or q.stride(0) % 8 or q.data_ptr() % 8:
+        if not lin.weight_scale.is_contiguous() or (INT8_WEIGHTS != "image" and (
+                q.dim() != 2 or q.stride(1) != 1 or q.stride(0) < q.shape[1] or q.stride(0) % 8 or q.data_ptr() % 8)):
             return False
     if lin.bias is not None and lin.bias.dtype != torch.float32:
         return False
@@ -420,7 +421,7 @@ def apply_linear(lin: nn.Module, x: torch.Tensor, *, norm: nn.LayerNorm | None =
         if (ops.small_linear_ok(M, N, K) and stats is None and small_ok(lin, x, compute, norm)
                 and out_dtype in (torch.float32, torch.bfloat16)
                 and (residual is None or (residual.dtype == out_dtype == torch.float32 and residual.dim() == 2
-                                          and residual.shape[1] == N and residual.stride(1) == 1))
+                                          and residual.shape[1] == N))
                 and (out is None or (out.dtype == out_dtype and out.is_contiguous()))):
             x2 = x.reshape(M, K)
             if x2.data_ptr() % 16 or x2.stride(1) != 1 or x2.stride(0) % 8:

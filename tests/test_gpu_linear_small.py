@@ -120,3 +120,37 @@ def test_float16_weights_at_few_rows(batch):
             assert torch.equal(blk(*args), ref(*args))
     w = torch.randn(64, 96, device=DEV).half()
     assert torch.equal(ops.frag_weight(w), ops.frag_weight(w.bfloat16()))
+
+
+def _lin(N, K, bias=True):
+    torch.manual_seed(N + K)
+    return torch.nn.Linear(K, N, bias=bias).to(DEV)
+
+
+@pytest.mark.parametrize("M", [2, 40])
+def test_expanded_rows_and_residual(M):
+    """Rows and residuals that share memory (expanded), of a stride below their width or of a transposed
+    matrix give what their copies give."""
+    from cortex.models._layers import apply_linear
+
+    K = N = 256
+    lin, norm = _lin(N, K), torch.nn.LayerNorm(K).to(DEV)
+    kw = dict(out_dtype=torch.float32, compute=torch.bfloat16)
+    views = [((1, K), lambda t: t.expand(M, K)), ((M + K,), lambda t: t.as_strided((M, K), (1, 1))),
+             ((K, M), lambda t: t.t()), ((M, 1, K), lambda t: t.expand(M, 3, K))]
+    with torch.no_grad():
+        for shape, view in views:
+            base = torch.randn(shape, device=DEV)
+            x, xb = view(base), view(base.bfloat16())
+            assert torch.equal(apply_linear(lin, xb, **kw), apply_linear(lin, xb.contiguous(), **kw))
+            assert torch.equal(apply_linear(lin, x, norm=norm, **kw), apply_linear(lin, x.contiguous(), norm=norm, **kw))
+        x = torch.randn(M, K, device=DEV).bfloat16()
+        for res in (torch.randn(1, N, device=DEV).expand(M, N), torch.randn(M + N, device=DEV).as_strided((M, N), (1, 1)),
+                    torch.randn(N, M, device=DEV).t()):
+            assert torch.equal(apply_linear(lin, x, residual=res, **kw), apply_linear(lin, x, residual=res.contiguous(), **kw))
+    from cortex.quantization.calibrate import QuantizedLinear
+
+    q8 = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=DEV)
+    scale = torch.rand(N, 2, device=DEV)[:, 0]  # every second value
+    got, want = (apply_linear(QuantizedLinear(q8, s, None), x, **kw) for s in (scale, scale.contiguous()))
+    assert ((got - want).norm() <= 1e-5 * want.norm())  # (another order of the K sums)
