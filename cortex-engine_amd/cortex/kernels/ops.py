@@ -775,8 +775,8 @@ def _plain_bf16_linear(x, weight, weight_scale, bias, act, residual, res_rows, o
     M = x.numel() // K
     if out is None:
         out = torch.empty((*x.shape[:-1], N), dtype=out_dtype, device=dev)
-    elif out.numel() != M * N:
-        raise ValueError("out must be row-major contiguous over its last dim")
+    elif out.numel() < M * N or out.numel() % max(N, 1):
+        raise ValueError(f"out must hold {M} rows of {N} values, got shape {tuple(out.shape)}")
     wp, xp, op, sp, bp, rp = (nat.ptr(t) for t in (weight, x, out, weight_scale, bias, residual))
     if (residual is not None and not ACT[act] and residual.dtype == out.dtype == torch.float32
             and (bias is None or bias.dtype == torch.float32)
@@ -841,6 +841,8 @@ def norm_linear(x: torch.Tensor, *, weight: torch.Tensor | None = None, weight_i
     out2 = out.reshape(-1, N)
     if out2.data_ptr() != out.data_ptr() or (M > 1 and out2.stride(0) < N) or out2.stride(-1) != 1:
         raise ValueError("out must be row-major contiguous over its last dim")
+    if out2.shape[0] < M:
+        raise ValueError(f"out must hold {M} rows of {N} values, got shape {tuple(out.shape)}")
     nrm = NORM[norm]
     if (nrm and stats is None and residual is None and compute_dtype == torch.bfloat16 and x2.dtype == torch.bfloat16
             and K % 64 == 0 and K <= 512 and N % 8 == 0 and out_dtype in (torch.bfloat16, torch.float32)

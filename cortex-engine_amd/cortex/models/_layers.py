@@ -422,7 +422,7 @@ def apply_linear(lin: nn.Module, x: torch.Tensor, *, norm: nn.LayerNorm | None =
                 and out_dtype in (torch.float32, torch.bfloat16)
                 and (residual is None or (residual.dtype == out_dtype == torch.float32 and residual.dim() == 2
                                           and residual.shape[1] == N))
-                and (out is None or (out.dtype == out_dtype and out.is_contiguous()))):
+                and (out is None or (out.dtype == out_dtype and out.is_contiguous() and out.numel() == M * N))):
             x2 = x.reshape(M, K)
             if x2.data_ptr() % 16 or x2.stride(1) != 1 or x2.stride(0) % 8:
                 x2 = x2.contiguous()

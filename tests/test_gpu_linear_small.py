@@ -154,3 +154,30 @@ def test_expanded_rows_and_residual(M):
     scale = torch.rand(N, 2, device=DEV)[:, 0]  # every second value
     got, want = (apply_linear(QuantizedLinear(q8, s, None), x, **kw) for s in (scale, scale.contiguous()))
     assert ((got - want).norm() <= 1e-5 * want.norm())  # (another order of the K sums)
+
+
+@pytest.mark.parametrize("M", [1, 30, 3000])
+def test_output_buffer_with_more_rows(M):
+    """An output of more rows than the result keeps the rest of its rows."""
+    from cortex.kernels import ops
+    from cortex.models._layers import apply_linear
+
+    K = N = 256
+    lin = _lin(N, K, bias=False)
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    with torch.no_grad():
+        for dtype in (torch.bfloat16, torch.float32):
+            want = apply_linear(lin, x, out_dtype=dtype, compute=torch.bfloat16)
+            out = torch.full((M + 5, N), 7.0, dtype=dtype, device=DEV)
+            apply_linear(lin, x, out_dtype=dtype, compute=torch.bfloat16, out=out)
+            assert (out[M:] == 7).all()
+            assert ((out[:M] - want).abs() <= 2.0 ** -7 * want.abs() + 1e-4).all()
+            w = lin.weight.bfloat16()
+            want = ops.norm_linear(x, weight=w, out_dtype=dtype)
+            out = torch.full((M + 5, N), 7.0, dtype=dtype, device=DEV)
+            ops.norm_linear(x, weight=w, out_dtype=dtype, out=out)
+            assert torch.equal(out[:M], want) and (out[M:] == 7).all()
+            with pytest.raises((ValueError, RuntimeError)):
+                ops.norm_linear(x, weight=w, out_dtype=dtype, out=out[:0])
+            with pytest.raises((ValueError, RuntimeError)):
+                ops.norm_linear(x, weight=lin.weight, out_dtype=dtype, out=out[:M - 1])
