@@ -24,10 +24,11 @@
 // and no column tile repeats the norm or the split.  Rows go in chunks that the caller's workspace
 // holds; the weight's planes are written with the first chunk.
 //
-// Not finite or not representable values: infinities and NaN go whole into the third part, which
-// only meets the other operand's first part, so inf * w keeps its sign (the other products see 0).
-// Values that round to infinity in bf16 are truncated instead.  Parts below 2^-126 are flushed by
-// the MFMA, as the fp32 product of such values mostly is.
+// Not finite values: an infinity is +-1 in its first part, 0 in the second and itself in the third, which
+// meets the other operand's first part only.  So inf * w is infinite with the right sign for every finite
+// w != 0 and for an infinite one (the third parts themselves never meet), and inf * 0 is NaN; a NaN goes
+// whole into the third part.  Values that round to infinity in bf16 are truncated instead.  Parts below 2^-126
+// are flushed by the MFMA, as the fp32 product of such values mostly is.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -60,11 +61,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // The three bf16 parts of v (p1 + p2 + p3 == v for every finite v above the underflow range).
 __device__ __forceinline__ void split3(float v, bf16& p1, bf16& p2, bf16& p3) {
   bf16 h = (bf16)v;
-  const uint32_t mag = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
-  if (mag >= 0x7f7f8000u) {  // rounds to infinity, or not finite
-    const uint32_t t = __builtin_bit_cast(uint32_t, v) & 0xffff0000u;
-    h = mag >= 0x7f800000u ? (bf16)0.0f : __builtin_bit_cast(bf16, (uint16_t)(t >> 16));
-  }
+  const uint32_t bits = __builtin_bit_cast(uint32_t, v), mag = bits & 0x7fffffffu;
+  if (mag >= 0x7f7f8000u)  // rounds to infinity, or not finite (+-1, see above)
+    h = __builtin_bit_cast(bf16, (uint16_t)(mag >= 0x7f800000u ? ((bits >> 16) & 0x8000u) | 0x3f80u : bits >> 16));
   const float r1 = v - (float)h;
   bf16 m = (bf16)r1;
   if (mag >= 0x7f800000u) m = (bf16)0.0f;

@@ -136,3 +136,19 @@ def test_split_linear_special_values(form):
         assert torch.equal(fn(got), fn(want))
     ok = torch.isfinite(want)
     assert ((got - want).abs()[ok] <= 2.0 ** -20 * want.abs()[ok]).all()
+
+
+def test_split_linear_infinities_that_meet():
+    """Infinities of x and of the weight at the same k: their signed product, as the fp32 product gives it."""
+    ops = _ops()
+    inf = float("inf")
+    x = torch.ones(4, 64, device=DEV)
+    x[0, 5], x[1, 5], x[2, 5], x[3, 5] = inf, -inf, 0.0, float("nan")
+    w = torch.full((16, 64), 0.5, device=DEV)
+    w[1, 5], w[2, 5], w[3, 5] = inf, -inf, 0.0
+    got = ops.norm_linear(x, weight=w, compute_dtype=torch.float32).cpu()
+    want = (x.cpu().double() @ w.cpu().double().t()).float()
+    for fn in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(fn(got), fn(want))
+    ok = torch.isfinite(want)
+    assert torch.equal(got[ok], want[ok])
