@@ -18,11 +18,11 @@
 //                 written in that order, so P goes from the score registers straight into the MFMA.
 // The tiles to visit are listed in LDS first: those with a key that the length and the key mask allow and,
 // with a tile mask (block_e a multiple of 64), that one of the workgroup's query tiles allows.
-// Infinities and NaN go whole into the third part, which meets only the other operand's first.
 #include <hip/hip_runtime.h>
 
 #include "attention.h"
 #include "common.h"
+#include "split_parts.h"
 
 namespace cortex {
 
@@ -35,29 +35,6 @@ constexpr int AS_BLK = 1024;      // one plane's block of 32 x 16 operand values
 constexpr int AS_V0 = 24 * AS_BLK;  // V planes behind the K planes
 constexpr float AS_RESCALE = 8.0f;  // log2 units by which a tile must raise the reference max to move it
 
-struct Parts {
-  bf16x8 p[3];
-};
-// the parts of 8 values; SPECIAL: they may be infinite, NaN or round to infinity
-template <bool SPECIAL>
-__device__ __forceinline__ Parts split8(const float (&v)[8]) {
-  Parts r;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    bf16 h = (bf16)v[j];
-    const uint32_t mag = __builtin_bit_cast(uint32_t, v[j]) & 0x7fffffffu;
-    if (SPECIAL && mag >= 0x7f7f8000u)
-      h = mag >= 0x7f800000u ? (bf16)0.0f
-                             : __builtin_bit_cast(bf16, (uint16_t)(__builtin_bit_cast(uint32_t, v[j]) >> 16));
-    const float r1 = v[j] - (float)h;
-    bf16 m = (bf16)r1;
-    if (SPECIAL && mag >= 0x7f800000u) m = (bf16)0.0f;
-    r.p[0][j] = h;
-    r.p[1][j] = m;
-    r.p[2][j] = (bf16)(r1 - (float)m);
-  }
-  return r;
-}
 __device__ __forceinline__ void put_parts(unsigned char* dst, const Parts& s) {
 #pragma unroll
   for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(dst + q * AS_BLK) = s.p[q];

@@ -93,3 +93,25 @@ def test_extremes(scale):
     assert torch.isposinf(got[:, 7]).all() and torch.isnan(got[:, 8]).all()
     rest = torch.cat([got[:, :7], got[:, 9:]], 1)
     assert torch.isfinite(rest).all()
+
+
+@pytest.mark.parametrize("L", [40, 8192])
+def test_infinite_operands(L):
+    """An infinite query component on an infinite key of the other sign is a score of -inf: that key drops out."""
+    from cortex.kernels import ops
+
+    g = torch.Generator(DEV).manual_seed(5)
+    q, k, v = (torch.randn(1, 4, n, 64, generator=g, device=DEV) for n in (L, 70, 70))
+    q[0, 0, :, 3] = float("inf")
+    k[0, 0, :, 3] = float("-inf")
+    k[0, 0, 5:9, 3] = 0.0  # inf * 0: NaN
+    q[0, 1, :, 3] = float("inf")
+    k[0, 1, :, 3] = float("-inf")
+    got = ops.attention(q, k, v)
+    assert torch.isnan(got[0, 0]).all()
+    assert (got[0, 1] == 0).all()  # every score -inf: no key counts
+    q[0, 1, 1:, 3] = 1.0
+    k[0, 1, :9, 3] = torch.randn(9, generator=g, device=DEV)
+    got = ops.attention(q[:, 1:2], k[:, 1:2], v[:, 1:2])
+    assert torch.isnan(got[0, 0, 0]).all() or L == 1
+    _check(got[:, :, 1:], q[:, 1:2, 1:], k[:, 1:2, :9], v[:, 1:2, :9], None)
