@@ -1,6 +1,7 @@
 // fp32 attention on the bf16 matrix cores for gfx950 (head dim 64): every fp32 operand -- queries, keys,
-// values and the probabilities -- as the exact sum of three bf16 parts, six products of order up to
-// 2^-16 each (exact, summed in fp32), as gemm_split.hip does for the linears; the softmax in fp32.
+// values and the probabilities -- as the exact sum of three bf16 parts (split_parts.h), six products of order up
+// to 2^-16 each (exact, summed in fp32), as gemm_split.hip does for the linears; the softmax in fp32, its
+// probabilities by the hardware's exp2 (0 below 2^-126, where the largest of a row is at least 1).
 //
 // What bounds it.  On the fp32 MFMA (157 TFLOP/s) a 32 x 64 block of scores and its P V cost 8192 cycles
 // of a SIMD; six bf16 products cost 3072 (v_mfma_f32_32x32x16_bf16).  Beside them a wavefront spends about

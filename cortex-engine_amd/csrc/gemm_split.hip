@@ -1,14 +1,18 @@
 // fp32 norm + linear on the bf16 matrix cores for gfx950:  y = epi( norm(x) . W^T ), fp32 in and out.
 //
-// An fp32 value is the exact sum of three bf16 values (3 x 8 significant bits, each part rounded
-// to nearest from what the parts before it leave).  A product of two fp32 operands is then the sum
-// of nine bf16 products, every one exact in fp32; the three of order 2^-24 and below (a2 w3, a3 w2,
+// An fp32 value is the exact sum of three bf16 values (split_parts.h).  A product of two fp32 operands is then
+// the sum of nine bf16 products, every one exact in fp32; the three of order 2^-24 and below (a2 w3, a3 w2,
 // a3 w3, unbiased: the parts' signs are independent) are left out, less than the rounding of one
 // fp32 addition.  An int8 weight is a bf16 value by itself: three products, none left out.  All sums
-// are fp32, in the MFMA accumulators, no more of them than on the fp32 MFMA (per 32 of K 6 or 12
-// accumulations of 16 products, against 8 of 4), and only the leading product's are large, so the
+// are fp32, in the MFMA accumulators: per 32 of K 6 accumulations of 16 products with an int8 weight and
+// 12 with an fp32 one, against 8 of 4 on the fp32 MFMA, but only the leading product's are large, so the
 // error against 64 bits is not larger (2-norm, N(0, 1) rows, fp32 MFMA -> here: K 512 4.0e-7 -> 2.1e-7
 // with an int8 weight, 3.4e-7 with an fp32 one; K 2048 8.1e-7 -> 4.2e-7 and 7.0e-7).
+//
+// At the bottom of the range it is larger: an operand value below 2^-110 is off by up to 2^-134, half of
+// bf16's smallest step (its parts are not flushed, but end there), where the fp32 MFMA kept its 24 bits.
+// N(0, 1) rows scaled by 2^-110: 1.7e-7, as unscaled; by 2^-114 5.8e-7, 2^-118 8.8e-6, 2^-126 2.2e-3 (the
+// fp32 MFMA 2.8e-7 throughout).  Beside values near 1 that is far below their rounding.
 //
 // What bounds it.  v_mfma_f32_16x16x4_f32 gives 157 TFLOP/s, v_mfma_f32_16x16x32_bf16 2.5 PFLOP/s:
 // six products of the latter are 2.6 times, three 5.3 times the former's rate.  The operand refill
@@ -23,16 +27,11 @@
 // direct-to-LDS transfers and its fragment reads are linear, without a swizzle or a bank conflict,
 // and no column tile repeats the norm or the split.  Rows go in chunks that the caller's workspace
 // holds; the weight's planes are written with the first chunk.
-//
-// Not finite values: an infinity is +-1 in its first part, 0 in the second and itself in the third, which
-// meets the other operand's first part only.  So inf * w is infinite with the right sign for every finite
-// w != 0 and for an infinite one (the third parts themselves never meet), and inf * 0 is NaN; a NaN goes
-// whole into the third part.  Values that round to infinity in bf16 are truncated instead.  Parts below 2^-126
-// are flushed by the MFMA, as the fp32 product of such values mostly is.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
 #include "gemm.h"
+#include "split_parts.h"
 
 namespace cortex {
 
@@ -57,20 +56,6 @@ __device__ __forceinline__ void lds_dma_1k(const unsigned char* src, uint32_t la
 
 constexpr int SP_BLK = 1024;  // bytes of one plane's 32 x 16 block
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// The three bf16 parts of v (p1 + p2 + p3 == v for every finite v above the underflow range).
-__device__ __forceinline__ void split3(float v, bf16& p1, bf16& p2, bf16& p3) {
-  bf16 h = (bf16)v;
-  const uint32_t bits = __builtin_bit_cast(uint32_t, v), mag = bits & 0x7fffffffu;
-  if (mag >= 0x7f7f8000u)  // rounds to infinity, or not finite (+-1, see above)
-    h = __builtin_bit_cast(bf16, (uint16_t)(mag >= 0x7f800000u ? ((bits >> 16) & 0x8000u) | 0x3f80u : bits >> 16));
-  const float r1 = v - (float)h;
-  bf16 m = (bf16)r1;
-  if (mag >= 0x7f800000u) m = (bf16)0.0f;
-  p1 = h;
-  p2 = m;
-  p3 = (bf16)(r1 - (float)m);
-}
 
 struct SplitArgs {
   int64_t M, N, K, KB;       // rows of this chunk, columns, depth, 32-K blocks
@@ -109,17 +94,9 @@ __device__ __forceinline__ float load_param(const void* p, int dtype, int64_t i)
 __device__ __forceinline__ void put_planes(unsigned char* dst, const float (&v)[16], int lane) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    bf16x8 p[3];
+    const Parts s = split8<true>(v + h * 8);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      bf16 a, b, c;
-      split3(v[h * 8 + j], a, b, c);
-      p[0][j] = a;
-      p[1][j] = b;
-      p[2][j] = c;
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(dst + (h * 3 + q) * SP_BLK + lane * 16) = p[q];
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(dst + (h * 3 + q) * SP_BLK + lane * 16) = s.p[q];
   }
 }
 

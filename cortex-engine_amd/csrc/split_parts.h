@@ -1,4 +1,5 @@
-// fp32 operands as exact sums of three bf16 parts, for products on the bf16 matrix cores (attention_split.hip).  The method: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence
+// fp32 operands as exact sums of three bf16 parts, for products on the bf16 matrix cores (gemm_split.hip,
+// attention_split.hip).  The method: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence
 // Datatype For Higher-Precision Computations" (ARITH 2019).
 //
 // Each part is the bf16 value nearest to what the parts before it leave: p1 + p2 + p3 == v while the third

@@ -152,3 +152,22 @@ def test_split_linear_infinities_that_meet():
         assert torch.equal(fn(got), fn(want))
     ok = torch.isfinite(want)
     assert torch.equal(got[ok], want[ok])
+
+
+@pytest.mark.parametrize("form", ["int8", "nk"])
+@pytest.mark.parametrize("power", [-100, -110, -114, -118, -126])
+def test_split_linear_smallest_values(form, power):
+    """Rows near the bottom of the range: full precision down to 2^-110, below that every operand value off
+    by at most 2^-134 (half of the smallest bf16 step)."""
+    ops = _ops()
+    g = torch.Generator(DEV).manual_seed(8)
+    x = torch.randn(64, 256, generator=g, device=DEV) * 2.0 ** power
+    kw, wd = _weight(ops, form, 128, 256, g)
+    want = x.double() @ wd.t().contiguous()
+    got = ops.norm_linear(x, **kw, compute_dtype=torch.float32)
+    step = 2.0 ** -149 * (1 + got.shape[1])  # (the sums' own denormals)
+    slack = 0 if power >= -100 else 2.0 ** -134 * wd.abs().sum(1)
+    rel = (12 * 9 + 16) * 2.0 ** -24 * (x.double().abs() @ wd.abs().t().contiguous())
+    assert ((got.double() - want).abs() <= rel + slack + step).all()
+    if power >= -110:
+        assert ((got.double() - want).norm() <= 4e-7 * want.norm())
