@@ -149,7 +149,17 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs a) {
       }
     }
   };
-  auto stage_tile = [&]() __attribute__((always_inline)) {
+  auto stage_tile = [&](int t) __attribute__((always_inline)) {
+    const int64_t rem = len - (int64_t)t * AS_KT;
+    if (rem < AS_KT) {  // rows past the end count as 0: their probability 0 times the last row's infinity is NaN
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int ku = wid * 2 + u;
+          if ((ku >> 1) * 16 + (j >> 2) * 8 + (ku & 1) * 4 + (j & 3) >= rem) vr[u][j] = 0.0f;
+        }
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int ku = wid * 2 + u;
@@ -167,7 +177,7 @@ __global__ __launch_bounds__(256, 2) void attention_split_kernel(AttnArgs a) {
   for (int i = 0; i < n; ++i) {
     const int t = wave_uniform((int)klist[i]);
     const uint64_t bits = (uint64_t)wave_uniform((int64_t)kmask[t]);
-    stage_tile();
+    stage_tile(t);
     const bool ok_q = bm_ok != 0;
     lds_barrier();
     if (i + 1 < n) load_tile(wave_uniform((int)klist[i + 1]));

@@ -115,3 +115,19 @@ def test_infinite_operands(L):
     got = ops.attention(q[:, 1:2], k[:, 1:2], v[:, 1:2])
     assert torch.isnan(got[0, 0, 0]).all() or L == 1
     _check(got[:, :, 1:], q[:, 1:2, 1:], k[:, 1:2, :9], v[:, 1:2, :9], None)
+
+
+@pytest.mark.parametrize("L", [40, 8192])
+@pytest.mark.parametrize("E", [1, 70, 150])
+def test_infinite_last_value(L, E):
+    """An infinite value in the last row, whose tile has rows past the end, stays infinite with its sign."""
+    from cortex.kernels import ops
+
+    g = torch.Generator(DEV).manual_seed(6)
+    q, k, v = (torch.randn(1, 4, n, 64, generator=g, device=DEV) for n in (L, E, E))
+    v[0, 0, -1, 7] = float("inf")
+    v[0, 1, -1, 8] = float("-inf")
+    got = ops.attention(q, k, v, scale=0.01)
+    assert torch.isposinf(got[0, 0, :, 7]).all() and torch.isneginf(got[0, 1, :, 8]).all()
+    got[0, 0, :, 7] = got[0, 1, :, 8] = 0
+    assert torch.isfinite(got).all()
