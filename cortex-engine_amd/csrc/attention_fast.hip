@@ -188,8 +188,11 @@ void attention_fast_kernel(AttnArgs a) {
   // V transfer of this lane: the same rows as K, row-major into the V stage with the vswz
   // chunk swizzle (lane i: row 8 wid + i / 8, stored chunk i % 8 = logical (i % 8) ^ vswz(row))
   const int64_t v_col = ((lane & 7) ^ vswz(k_row)) * 8;
+  // With a key mask the resource ends with the sample's last row, and rows past it are read from behind that
+  // end, as zeros: their probability of 0 times an infinity of a clamped row would be NaN.
+  const uint32_t v_end = KM ? (uint32_t)((max(len, (int64_t)1) - 1) * a.v_sl * 2 + 128) : 0xffffffffu;
   const __amdgpu_buffer_rsrc_t v_rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(Vb), (short)0, (int)0xffffffffu, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(Vb), (short)0, (int)v_end, 0x00020000);
 
   auto k_stage = [&](int j) { return smem + j * AF_KTILE; };
   auto v_stage = [&](int j) { return smem + AF_CH * AF_KTILE + j * AF_VTILE; };
@@ -274,6 +277,7 @@ void attention_fast_kernel(AttnArgs a) {
       const int64_t kr = min(k0 + k_row, len - 1);
       koff = (uint32_t)((kr * a.k_sl + k_col) * 2);
       voff = (uint32_t)((kr * a.v_sl + v_col) * 2);
+      if (KM && k0 + k_row >= len) voff = v_end;
     }
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         k_rsrc, (__attribute__((address_space(3))) void*)(k_stage(j) + wid * 1024), 16, (int)koff, 0, 0, 0);
@@ -342,7 +346,7 @@ void attention_fast_kernel(AttnArgs a) {
       if (__any(mx * sl > m_run[qg] + RESCALE)) {
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_tile = mx * sl;  // finite: every tile holds at least one valid key
+        const float m_tile = mx * sl;  // (every tile holds at least one valid key)
         if (m_run[qg] == -INFINITY) {
           m_run[qg] = m_tile;
         } else {
@@ -355,12 +359,14 @@ void attention_fast_kernel(AttnArgs a) {
           for (int t = 0; t < 4; ++t) o_acc[qg][t] *= alpha;
         }
       }
+      // (with a key mask, every allowed key of the tiles so far may score -inf)
+      const float ref = KM && m_run[qg] == -INFINITY ? 0.0f : m_run[qg];
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[qg][2 * c][i], sl, -m_run[qg]));  // -inf -> 0
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(s[qg][2 * c + 1][i], sl, -m_run[qg]));
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[qg][2 * c][i], sl, -ref));  // -inf -> 0
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(s[qg][2 * c + 1][i], sl, -ref));
           if constexpr (KM) l_sum[qg] += p0 + p1;
           pf[qg][c][i] = (bf16)p0;
           pf[qg][c][4 + i] = (bf16)p1;

@@ -182,3 +182,31 @@ def test_key_mask_precision_of_the_general_kernel(B, L, E, amp):
     fast = (ops.attention(q, k, v, key_mask=m) - want).norm()
     general = (ops.attention(q, k, v, key_mask=m, block_mask=tiles, block_l=1, block_e=1) - want).norm()
     assert fast <= 1.002 * general
+
+
+@pytest.mark.parametrize("B,L", [(1, 40), (64, 256)])
+@pytest.mark.parametrize("E", [70, 130, 200, 330])
+def test_key_mask_infinite_operands(B, L, E):
+    """Per-key masks: an infinite value in the last row stays infinite although the tile's other rows lie past
+    the end, and a first tile whose allowed keys all score -inf leaves the rest of the row as it is."""
+    from cortex.kernels import ops
+
+    g = torch.Generator().manual_seed(B + E)
+    q, k, v = ((torch.randn(B, 4, n, DH, generator=g) / 2).bfloat16() for n in (L, E, E))
+    m = torch.rand(B, E, generator=g) < 0.6
+    m[:, 3], m[:, 64:128], m[:, -1] = True, True, True
+    q[:, :, :, 2] = 1.0
+    v[:, 0, -1, 7] = float("inf")
+    v[:, 1, -1, 7] = float("-inf")
+    k[:, 2, :64, 2] = float("-inf")
+    k[:, 3, :, 2] = float("-inf")
+    v[:, 0, 64:128, 8] = float("inf")  # (the fifth tile takes the second's place on chip)
+    got = ops.attention(q.to(DEV), k.to(DEV), v.to(DEV), key_mask=m.to(DEV), scale=0.05).float().cpu()
+    assert torch.isposinf(got[:, 0, :, 7:9]).all() and torch.isneginf(got[:, 1, :, 7]).all()
+    assert torch.isfinite(got[:, :2, :, :7]).all() and (got[:, 3] == 0).all()
+    for b in {0, B - 1}:
+        mb = m[b].clone()
+        mb[:64] = False
+        ref = O.attention_bruteforce_f64(q[b:b + 1, 2:3].float(), k[b:b + 1, 2:3][:, :, mb].float(),
+                                         v[b:b + 1, 2:3][:, :, mb].float(), scale=0.05)
+        _close(got[b:b + 1, 2:3].numpy(), ref)
