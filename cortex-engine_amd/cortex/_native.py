@@ -82,6 +82,7 @@ _SIGNATURES = {
         [_i64, _i64, _i64, _int, _ptr, _i64, _int, _ptr, _ptr, _ptr, _int, _int, _int, _int, _ptr, _i64, _ptr,
          _int, _ptr, _int, _int, _ptr, _i64, _i64, _int, _ptr, _i64, _ptr],
     ),
+    "cortex_bf16_gemm_form": (_int, [_i64, _i64, _i64, _int, _int]),
     "cortex_linear_small": (
         _int,
         [_i64, _i64, _i64, _int, _ptr, _i64, _ptr, _ptr, _f32, _int, _ptr, _i64, _ptr, _ptr, _int, _ptr, _i64, _i64, _int,

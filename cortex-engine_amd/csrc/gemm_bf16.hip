@@ -773,14 +773,19 @@ __global__ __launch_bounds__(512) void gemm_persist_kernel(GemmArgs g) {
   }
 }
 
+// Past one wave of 256 x 256 tiles, with bf16 out.
+bool persist_ok(const GemmArgs& g) {
+  const int64_t ntiles = cdiv(g.M, 256) * (g.N / 256);
+  if (g.N % 256 != 0 || ntiles <= cu_count() || cu_count() < 8) return false;
+  // 32-bit transfer offsets (the scalar-base form) address both operands, 32-bit element
+  // offsets the output; larger tensors take the one-tile-per-workgroup kernel
+  return g.M * g.ld_x * 2 < (1LL << 32) && g.N * g.ld_w * 2 < (1LL << 32) && g.M * g.ld_out * 2 < (1LL << 32) &&
+         ntiles <= 0x7fffffffLL;
+}
+
 template <int ACT>
 int launch_persist(const GemmArgs& g, hipStream_t stream) {
   const int64_t ntiles = cdiv(g.M, 256) * (g.N / 256);
-  // 32-bit transfer offsets (the scalar-base form) address both operands, 32-bit element
-  // offsets the output; larger tensors take the one-tile-per-workgroup kernel
-  if (g.M * g.ld_x * 2 >= (1LL << 32) || g.N * g.ld_w * 2 >= (1LL << 32) || g.M * g.ld_out * 2 >= (1LL << 32) ||
-      ntiles > 0x7fffffffLL)
-    return 0;
   const int G = (int)std::min<int64_t>(ntiles, cu_count() & ~7);
   hipLaunchKernelGGL((gemm_persist_kernel<ACT>), dim3((unsigned)G), dim3(512), 0, stream, g);
   CORTEX_CHECK_LAUNCH("gemm_persist_kernel");
@@ -991,13 +996,16 @@ int launch_res_dw_impl(const GemmArgs& g, hipStream_t stream) {
 
 // Tile by shape.  A launch takes whole rounds: one tile of 256 x 256 or 256 x 192 per CU and round (a round with a few
 // tiles costs what a full one does), 128 x 128 ones two to a CU.  In rounds of 256 x 256 tiles a round of 256 x 192
-// takes 0.73 (K = 512) to 0.84, one 128 x 128 tile per CU 0.45 .. 0.57, two 0.69 .. 0.82, more 0.40 + 0.27 per CU's worth;
-// the least of the three (past three rounds the persistent 256 x 256 tiles lead again).  Measured, us (fill a CU
-// nearly once, else 128 x 128 -> this rule): 3072 x 3072 x 768 GELU 29.0 -> 21.6, 4096 x 2304 x 768 26.3 -> 19.8, 9216 x
-// 2304 x 768 51.1 -> 42.0, 6144 x 1536 x 512 19.3 -> 14.5, 12288 x 1536 x 512 34.7 -> 28.8, 9216 x 2048 x 512 GELU 38.9 -> 32.5,
-// 12288 x 768 x 256 13.3 -> 9.9, 4608 x 2048 x 512 GELU 22.2 -> 19.6.
+// takes 0.73 (K = 512) to 0.84, one 128 x 128 tile per CU 0.45 .. 0.57, two 0.69 .. 0.82, and more of them 0.40 + 0.27 to
+// 0.35 per CU's worth, the more the longer K is, and with int8 weights, which every tile widens anew, 0.03 on top.  The
+// least of the three.  Measured, us: few rounds (fill a CU nearly once, else 128 x 128 -> this rule) 3072 x 3072 x 768
+// GELU 29.0 -> 21.6, 4096 x 2304 x 768 26.3 -> 19.8, 9216 x 2304 x 768 51.1 -> 42.0, 6144 x 1536 x 512 19.3 -> 14.5, 12288 x
+// 768 x 256 13.3 -> 9.9, 4608 x 2048 x 512 GELU 22.2 -> 19.6; many (128 x 128 / 256 x 256 tiles) 16384 x 2048 x 512 GELU
+// 48.5 / 40.8, 30000 x 2304 x 768 140 / 132, 36864 x 2304 x 768 157 / 138, and where the last round is a few tiles, 33000 x
+// 1024 x 512 50.4 / 57.7, 33000 x 1024 x 256 GELU 40.4 / 45.0; int8 weights 9216 x 2048 x 512 GELU 39.6 / 42.6, 24576 x 1536 x
+// 512 59.7 / 56.2, 28160 x 3072 x 768 GELU 208 / 167.
 enum TileChoice { T128 = 0, T256 = 4, T192 = 6, T128_K2 = 7 };
-TileChoice wide_tile(const GemmArgs& g, bool allow192) {
+TileChoice wide_tile(const GemmArgs& g, bool w8) {
   const int ncu = cu_count();
   const int64_t t256 = cdiv(g.M, 256) * cdiv(g.N, 256), t192 = cdiv(g.M, 256) * cdiv(g.N, 192);
   const int64_t t128 = cdiv(g.M, 128) * cdiv(g.N, 128);
@@ -1005,8 +1013,9 @@ TileChoice wide_tile(const GemmArgs& g, bool allow192) {
   // the first round follow one another without one
   const double c256 = (double)cdiv(t256, ncu);
   const int64_t r192 = cdiv(t192, ncu);
-  const double c192 = allow192 && g.N % 192 == 0 && r192 <= 3 ? 0.82 * r192 : 1e30;
-  const double c128 = t128 <= ncu ? 0.48 : t128 <= 2 * ncu ? 0.76 : 0.40 + 0.27 * t128 / ncu;
+  const double c192 = !w8 && g.N % 192 == 0 && r192 <= 3 ? 0.82 * r192 : 1e30;
+  const double per_cu = 0.27 + 0.01 * (double)g.K / 256 + (w8 ? 0.03 : 0.0);  // (K 256 .. 768 measured)
+  const double c128 = t128 <= ncu ? 0.48 : t128 <= 2 * ncu ? 0.76 : 0.40 + per_cu * t128 / ncu;
   if (c128 < c256 && c128 < c192) return T128;
   return c192 < c256 ? T192 : T256;
 }
@@ -1016,17 +1025,13 @@ int dispatch(const GemmArgs& g, hipStream_t stream) {
   if constexpr (sizeof(TW) == 1) {
     // int8 weights (widened at the fragment read): the same tiles as bf16 weights but the
     // 192-column one
-    return wide_tile(g, false) == T256 ? launch<B256x256s2w, ACT, RES, TOUT, bf16, TW>(g, stream)
+    return wide_tile(g, true) == T256 ? launch<B256x256s2w, ACT, RES, TOUT, bf16, TW>(g, stream)
                                        : launch<B128x128s2, ACT, RES, TOUT, bf16, TW>(g, stream);
   } else {
-    switch (wide_tile(g, true)) {
+    switch (wide_tile(g, false)) {
       case T256:
-        // past one wave of 256 x 256 tiles, bf16 out: persistent tiles (see gemm_persist_kernel)
         if constexpr (!RES && sizeof(TOUT) == 2) {
-          if (g.N % 256 == 0 && cdiv(g.M, 256) * (g.N / 256) > cu_count() && cu_count() >= 8) {
-            const int st = launch_persist<ACT>(g, stream);
-            if (st != 0) return st;
-          }
+          if (persist_ok(g)) return launch_persist<ACT>(g, stream);
         }
         return launch<B256x256s2, ACT, RES, TOUT>(g, stream);
       case T192: return launch<B256x192s2, ACT, RES, TOUT>(g, stream);
@@ -1041,7 +1046,7 @@ int dispatch(const GemmArgs& g, hipStream_t stream) {
 // 128 x 128 workgroup per CU the K split of the residual GEMMs.
 template <int ACT, class TOUT>
 int dispatch_rs(const GemmArgs& g, hipStream_t stream) {
-  TileChoice t = wide_tile(g, true);
+  TileChoice t = wide_tile(g, false);
   // at most one 128 x 128 workgroup per CU: K split over two wave groups (eight wavefronts)
   if (t == T128 && g.K % 128 == 0 && cdiv(g.M, 128) * cdiv(g.N, 128) <= cu_count()) t = T128_K2;
   switch (t) {
@@ -1604,6 +1609,21 @@ int try_gemm_bf16(const GemmArgs& g, int x_dtype, int w_dtype, int w_layout, int
 }  // namespace cortex
 
 using namespace cortex;
+
+extern "C" int cortex_bf16_gemm_form(int64_t M, int64_t N, int64_t K, int w_dtype, int out_dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 || N % 8 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+  if ((w_dtype != DT_BF16 && w_dtype != DT_I8) || (out_dtype != DT_BF16 && out_dtype != DT_F32)) return 0;
+  GemmArgs g = {};
+  g.M = M;
+  g.N = N;
+  g.K = g.ld_x = g.ld_w = K;
+  g.ld_out = N;
+  switch (wide_tile(g, w_dtype == DT_I8)) {
+    case T256: return w_dtype == DT_BF16 && out_dtype == DT_BF16 && persist_ok(g) ? 4 : 3;
+    case T192: return w_dtype == DT_I8 ? 1 : 2;
+    default: return 1;
+  }
+}
 
 extern "C" int cortex_linear_w8a8(int64_t M, int64_t N, int64_t K, const int8_t* x, int64_t ld_x, float a_scale,
                                   const int8_t* w, int64_t ld_w, const float* w_scale, const float* bias, int act,

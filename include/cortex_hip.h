@@ -253,6 +253,11 @@ int cortex_norm_linear(int64_t M, int64_t N, int64_t K, int x_dtype, const void*
                        int64_t ld_res, int64_t res_rows, int out_dtype, void* out, int64_t ld_out,
                        hipStream_t stream);
 
+/* The tiling that cortex_norm_linear takes for bf16 rows without a norm or a residual (contiguous, aligned;
+ * w_dtype 1 or 3, out_dtype 0 or 1): 1 128 x 128, 2 256 x 192, 3 256 x 256, 4 persistent 256 x 256; 0 where the
+ * tiled GEMM does not apply.  Launches nothing (without a GPU, the rule for 256 CUs). */
+int cortex_bf16_gemm_form(int64_t M, int64_t N, int64_t K, int w_dtype, int out_dtype);
+
 /* A bf16 linear with few rows in one launch (the chains of SelfAttentionBlock and
  * CrossAttentionBlock, cortex/models/perceiver.py:67-68,113-125, at one to a few samples):
  *   out = act((a . w^T) * w_scale + bias) + residual[m % res_rows]

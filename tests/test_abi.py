@@ -98,6 +98,35 @@ def test_invalid_arguments_return_status_and_message():
     assert rc == -1 and b"K = 256 or 512" in lib.cortex_last_error()
 
 
+# (rows, columns, K, int8 weight, tiling): 1 128 x 128, 2 256 x 192, 3 256 x 256, 4 persistent 256 x 256, the
+# faster one of its row where they were timed
+@pytest.mark.parametrize("M,N,K,w8,form", [
+    (3072, 3072, 768, False, 2), (4096, 2304, 768, False, 2), (4608, 2048, 512, False, 3), (2048, 2048, 512, False, 1),
+    (9216, 2304, 768, False, 2), (16384, 2304, 768, False, 2), (24576, 2304, 768, False, 4), (36864, 2304, 768, False, 4),
+    (16384, 2048, 512, False, 4), (33792, 2048, 512, False, 4), (18000, 3072, 768, False, 4), (45000, 1536, 512, False, 4),
+    (33000, 1024, 512, False, 1), (33000, 1024, 256, False, 1), (8192, 2048, 512, False, 3),
+    (9216, 2048, 512, True, 1), (16384, 2304, 768, True, 3), (24576, 1536, 512, True, 3), (33792, 2048, 512, True, 3),
+    (84480, 1024, 512, True, 3), (12288, 1536, 512, True, 1), (6144, 1536, 512, True, 3),
+    # with more tiles than CUs and N / 256 that does not divide the tile step
+    (26000, 1280, 128, False, 4), (33000, 2304, 128, False, 4), (64000, 768, 128, False, 4),
+])
+def test_bf16_gemm_tiling_by_shape(M, N, K, w8, form):
+    from cortex import _native as nat
+
+    assert nat.load().cortex_bf16_gemm_form(M, N, K, nat.I8 if w8 else nat.BF16, nat.BF16) == form
+
+
+def test_bf16_gemm_tiling_outside_its_form():
+    from cortex import _native as nat
+
+    lib = nat.load()
+    assert lib.cortex_bf16_gemm_form(0, 64, 64, nat.BF16, nat.BF16) == 0
+    assert lib.cortex_bf16_gemm_form(64, 64, 32, nat.BF16, nat.BF16) == 0
+    assert lib.cortex_bf16_gemm_form(64, 64, 64, nat.F32, nat.BF16) == 0
+    assert lib.cortex_bf16_gemm_form(64000, 768, 128, nat.BF16, nat.F32) == 3  # fp32 out: one tile a workgroup
+    assert lib.cortex_bf16_gemm_form(4_000_000, 768, 768, nat.BF16, nat.BF16) == 3  # rows past 4 GiB
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     import importlib
 
