@@ -30,6 +30,17 @@ def test_large_linear_column_parameters(M, N, K, act):
     assert ((got.double() - want).abs().amax() <= 2.0 ** -8 * want.abs().amax() + 2.0 ** -8)
 
 
+@pytest.mark.parametrize("M,N,K", [(26000, 1280, 128), (33000, 2304, 128), (64000, 768, 128), (15000, 3072, 256)])
+@pytest.mark.parametrize("act", [None, "gelu"])
+def test_persistent_linear_column_parameters(M, N, K, act):
+    """The same where the persistent tiles take the call (N / 256 = 5, 9, 3, 12 does not divide the tile step of
+    32, so that the next tile of a workgroup has other columns)."""
+    from cortex import _native as nat
+
+    assert nat.load().cortex_bf16_gemm_form(M, N, K, nat.BF16, nat.BF16) == 4
+    test_large_linear_column_parameters(M, N, K, act)
+
+
 @pytest.mark.parametrize("M,N,K", [(65536, 256, 2048), (65300, 256, 2112), (32769, 512, 2048), (21900, 768, 3072),
                                    (98400, 256, 2048)])
 @pytest.mark.parametrize("res_rows", [0, 384])
@@ -80,11 +91,12 @@ def test_tall_residual_layer_norm_equals_ring(M, N, K, res_rows):
 
 
 @pytest.mark.parametrize("M,N", [(3069, 2304), (4093, 2304), (6141, 2304), (7679, 2304), (9213, 2304), (4605, 2048),
-                                 (12285, 768), (12285, 1536), (9213, 2048), (16381, 2304)])
+                                 (12285, 768), (12285, 1536), (9213, 2048), (16381, 2304), (16381, 2048), (24573, 2304),
+                                 (33001, 1024)])
 @pytest.mark.parametrize("form", ["image", "int8", "rms"])
 def test_tile_rule(M, N, form):
-    """Row counts on every side of the tile rule (128 x 128, 256 x 192 and 256 x 256 tiles in one to three
-    rounds), partial last tiles: sampled and last rows against 64 bits, 2^-8."""
+    """Row counts on every side of the tile rule (128 x 128, 256 x 192 in one to three rounds, 256 x 256 in one
+    to four), partial last tiles: sampled and last rows against 64 bits, 2^-8."""
     from cortex.kernels import ops
     from cortex.kernels.fused_rmsnorm import norm_linear_int8
 
@@ -108,3 +120,17 @@ def test_tile_rule(M, N, form):
         want = torch.nn.functional.gelu(want)
     err = (got[rows].double() - want).abs()
     assert (err.norm() <= 2.0 ** -8 * want.norm()) and (err.amax() <= 2.0 ** -7 * want.abs().amax())
+
+
+def test_tile_rule_shapes_take_every_tiling():
+    """The shapes of ``test_tile_rule`` reach each tiling, the large ones in more than one round."""
+    from cortex import _native as nat
+
+    shapes = next(m for m in test_tile_rule.pytestmark if m.args[0] == "M,N").args[1]
+    rounds = {}
+    for M, N in shapes:
+        form = nat.load().cortex_bf16_gemm_form(M, N, 128, nat.BF16, nat.BF16)
+        width = {1: 128, 2: 192, 3: 256, 4: 256}[form]
+        tiles = -(-M // (128 if form == 1 else 256)) * -(-N // width)
+        rounds.setdefault(form, set()).add(-(-tiles // (512 if form == 1 else 256)))
+    assert set(rounds) == {1, 2, 3, 4} and {1, 2, 3} <= rounds[2] and max(rounds[4]) >= 4 and max(rounds[1]) >= 4
