@@ -303,7 +303,7 @@ int try_attention_split(const AttnArgs& a, int dtype, hipStream_t stream) {
   const int64_t nbh = a.B * a.H, nq = cdiv(a.Lq, 128);
   if (nbh > 65535 || cdiv(a.Lq, 64) * nbh > 0x7fffffffLL) return 0;
   // 128 queries a workgroup (K and V split once per 128 queries) once that gives every CU one
-  if (nq * nbh >= 256) {
+  if (nq * nbh >= cu_count()) {
     hipLaunchKernelGGL((attention_split_kernel<1>), dim3((unsigned)nq, (unsigned)nbh), dim3(256), 0, stream, a);
   } else {
     hipLaunchKernelGGL((attention_split_kernel<2>), dim3((unsigned)cdiv(a.Lq, 64), (unsigned)nbh), dim3(256), 0, stream,

@@ -65,6 +65,9 @@ __device__ __forceinline__ void mfma_16x16x32(f32x4& acc, const Frag<float>& a, 
   for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[j], b.v[j], acc, 0, 0, 0);
 }
 
+// CUs of the device that the first call finds current (256 where there is none; gemm_bf16.hip).
+int cu_count();
+
 // Output stores written through the L2 to memory at device scope (SC1).  A kernel's outputs
 // are read by the next kernel, mostly on other XCDs; written through as they are produced,
 // they leave no dirty lines behind for the L2 write-back at the end of the kernel, which

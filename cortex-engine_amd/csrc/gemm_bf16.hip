@@ -531,17 +531,6 @@ using B128x128s2k2 = BTile<128, 128, 2, 2, 2, 2>;
 using B256x256s2w = BTile<256, 256, 2, 2, 4>;
 using B128x128s2k2w = BTile<128, 128, 2, 1, 4, 2>;
 
-int cu_count() {
-  static int v = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
-  return v;
-}
-
 // ---------------------------------------------------------------------------------------
 // Persistent 256 x 256 tiles for bf16-output GEMMs past one wave of tiles (MLP-up with its
 // GELU and the kv projection at B >= 64; bf16 rows and bf16 weight rows, N % 256 == 0).
@@ -1550,6 +1539,17 @@ int dispatch_norm(const NormGemmArgs& a, hipStream_t stream) {
 }
 
 }  // namespace
+
+int cu_count() {
+  static int v = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    return n;
+  }();
+  return v;
+}
 
 int split_k_partials(const GemmArgs& g, int splits, hipStream_t stream) {
   using TL = B128x128s2;

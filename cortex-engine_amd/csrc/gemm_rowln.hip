@@ -558,7 +558,7 @@ int residual_ln(const char* who, int64_t M, int64_t N, int64_t K, const void* x,
     // 64 rows a workgroup past one workgroup of 32 per CU: the weight is streamed once per workgroup, and 32-row
     // ones would come in rounds (N = K = 512: 8704 rows 28.5 -> 21.4 us, 16384 32.8 -> 27.2, 32768 60.5 -> 53.8,
     // 65536 129.3 -> 128.6; 256: 8448 12.9 -> 10.3, 32768 25.2 -> 25.3)
-    const bool tall = M > 256 * RL_BM;
+    const bool tall = M > (int64_t)cu_count() * RL_BM;
 #define RL_DW(BN_, NK_)                                                                                           \
   do {                                                                                                            \
     if (q8) hipLaunchKernelGGL((gemm_rowln_dw_kernel<BN_, NK_, true>), grid, dim3(RL_THREADS), 0, stream, a);   \

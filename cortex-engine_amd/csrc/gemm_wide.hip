@@ -252,7 +252,8 @@ int try_gemm_wide(const GemmArgs& g, hipStream_t stream) {
   // long K (at 1024 the two forms are equal, 57 us at 65500 x 256) and rounds of tiles that fill the CUs: a last round
   // of an eighth costs what it would full (24576 x 768 x 3072, 288 tiles: 163 us in the other form, 180 here)
   const int64_t tiles = cdiv(g.M, GW_T) * (g.N / GW_T);
-  if (g.K < 2048 || tiles > 0x3fffffff || tiles < 256 || tiles * 4 < cdiv(tiles, 256) * 256 * 3) return 0;
+  const int64_t ncu = cu_count();
+  if (g.K < 2048 || tiles > 0x3fffffff || tiles < ncu || tiles * 4 < cdiv(tiles, ncu) * ncu * 3) return 0;
   if (g.M * g.ld_x * 2 > 0xffffffffll || g.N * g.ld_w * 2 > 0xffffffffll) return 0;
   WideArgs a = {};
   a.M = (int)g.M;
@@ -271,7 +272,7 @@ int try_gemm_wide(const GemmArgs& g, hipStream_t stream) {
   a.ld_out = g.ld_out;
   a.nt = (int)(g.N / GW_T);
   a.tiles = (int)tiles;
-  hipLaunchKernelGGL(gemm_wide_kernel, dim3(256), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(gemm_wide_kernel, dim3((unsigned)ncu), dim3(256), 0, stream, a);
   CORTEX_CHECK_LAUNCH("gemm_wide_kernel");
   return 1;
 }
