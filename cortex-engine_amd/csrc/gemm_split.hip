@@ -19,7 +19,7 @@
 // of a 128 x 128 tile is 48 KiB (24 + 8 with an int8 weight) per 96 (48) MFMAs of a wavefront, half
 // of a bf16 GEMM's per MFMA, since every fragment read from LDS is used up to six times.  The matrix
 // cores, throttled by power, give 1.83 PFLOP/s on random data (a loop of MFMAs on registers); at 8192 x
-// 512 x 2048 this kernel runs at 1.2 PFLOP/s of bf16 products with an fp32 weight, 1.0 with int8.
+// 512 x 2048 this kernel runs at 1.2 PFLOP/s of bf16 products with an fp32 weight, with int8 and a residual at 0.83.
 //
 // Two launches.  split_prep_kernel applies the norm (statistics computed on the spot) and writes
 // the parts of the rows and of the weight as planes in MFMA fragment order: per 32 rows and 16 of
@@ -546,23 +546,31 @@ int cortex_norm_linear_split(int64_t M, int64_t N, int64_t K, const float* x, in
     CORTEX_CHECK_LAUNCH("split_prep_kernel");
     const int64_t tiles = cdiv(g.M, 128) * cdiv(N, 128);
     CORTEX_CHECK_ARG(cdiv(g.M, 64) * cdiv(N, 64) <= 0x7fffffffLL, "cortex_norm_linear_split: N too large for the grid");
-    // 128 x 128 tiles from one per CU on: below that 64 x 64 ones fill more of the chip and their shorter
-    // steps hide less (3072 x 768 x 3072, 144 large tiles: equal).  Int8: two workgroups a CU with two
-    // stages each (8192 x 2048 x 512: 54 us, one with four 71), except where there is one tile per CU
-    // (8192 x 512 x 2048: four stages 51 us, two 58).  fp32: 144 KiB, one workgroup a CU; small tiles
-    // take a fourth stage while one workgroup a CU is all there is (256 x 512 x 2048: 31 us against 33 in
-    // all; 1024 x 1536 x 512 with two a CU: 28 against 31).
+    // Tile by shape (whole calls, us; 128 x 128 / 64 x 64).  64 x 64 tiles fill more of the chip while 128 x 128 ones
+    // are at most one per CU, and just above, where those start a second round; from there on 128 x 128 ones,
+    // which refill half as much per MFMA.  Their epilogue reads 64 residual values a lane with nothing beside
+    // it, so with a residual the line lies higher.
+    //   int8 (128 x 128 with two stages, two workgroups a CU).  At 256, 288, 320 and 384 tiles: 8192 .. 12288 x 512 x
+    //   512 31.0 / 28.2, 36.5 / 32.8, 38.5 / 34.2, 42.8 / 42.6, with a residual 44.5 / 31.0, 46.3 / 37.1, 46.9 / 37.8, 47.4 / 41.0 and
+    //   53.3 / 51.8 at 512; x 512 x 2048 86.1 / 90.7, 110 / 104, 114 / 114, 130 / 137, with a residual 101 / 87, 115 / 101, 120 /
+    //   108, 134 / 132 and 175 / 214 at 512.
+    //   fp32 (144 KiB, one workgroup a CU).  K = 512 43.7 / 41.8, 60.7 / 46.3 (280), 61.7 / 48.0, 66.2 / 56.6, with a residual
+    //   54.0 / 41.3, 79.1 / 46.1, 81.4 / 47.3, 86.8 / 53.3; K = 2048 122 / 129, 183 / 148 (280), 191 / 159, 206 / 191, with a residual
+    //   129 / 124, 202 / 143, 207 / 152, 224 / 189 and 260 / 272 at 512; without one, from 7/8 of the CUs on 2048 x 2048 x
+    //   512 40.8 / 50.1, 16384 x 256 x 256 34.0 / 33.5, 4096 x 1024 x 2048 109 / 118.  64 x 64 take a fourth stage while one
+    //   workgroup a CU is all there is (256 x 512 x 2048: 31 against 33; 1024 x 1536 x 512 with two a CU: 31 against 28).
     // The fp32 MFMA kernel before, whole call with the norm: 8192 x 2048 x 512 273 us -> 69 (int8), 314 ->
     // 125 (fp32, (K, N)); 256 x 512 x 2048 without 178 -> 22 and 232 -> 31; 64 x 256 x 256 62 -> 10.
+    const int64_t ncu = cu_count(), line = residual ? ncu * 3 / 2 : ncu * 5 / 4;
     int rc;
     if (w_dtype == DT_I8)
-      rc = tiles > 256    ? launch_split<SplitTile<128, 128, 1, 2, 2>>(g, stream)
-           : tiles == 256 ? launch_split<SplitTile<128, 128, 1, 4, 1>>(g, stream)
-                          : launch_split<SplitTile<64, 64, 1, 4, 2>>(g, stream);
+      rc = tiles > line ? launch_split<SplitTile<128, 128, 1, 2, 2>>(g, stream)
+                        : launch_split<SplitTile<64, 64, 1, 4, 2>>(g, stream);
+    else if (tiles > line || (!residual && tiles > ncu * 7 / 8 && tiles <= ncu))
+      rc = launch_split<SplitTile<128, 128, 3, 3, 1>>(g, stream);
     else
-      rc = tiles >= 256                                ? launch_split<SplitTile<128, 128, 3, 3, 1>>(g, stream)
-           : cdiv(g.M, 64) * cdiv(N, 64) > 256         ? launch_split<SplitTile<64, 64, 3, 3, 2>>(g, stream)
-                                                       : launch_split<SplitTile<64, 64, 3, 4, 1>>(g, stream);
+      rc = cdiv(g.M, 64) * cdiv(N, 64) > ncu ? launch_split<SplitTile<64, 64, 3, 3, 2>>(g, stream)
+                                             : launch_split<SplitTile<64, 64, 3, 4, 1>>(g, stream);
     if (rc != OK) return rc;
   }
   return OK;

@@ -171,3 +171,22 @@ def test_split_linear_smallest_values(form, power):
     assert ((got.double() - want).abs() <= rel + slack + step).all()
     if power >= -110:
         assert ((got.double() - want).norm() <= 4e-7 * want.norm())
+
+
+@pytest.mark.parametrize("form", ["int8", "nk"])
+@pytest.mark.parametrize("M,N,K", [(7424, 512, 2048), (1661, 2048, 2075), (1920, 2048, 96), (2049, 2048, 96), (2049, 2048, 1056),
+                                   (2600, 2050, 96), (3201, 2048, 96)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_split_linear_tile_rule(form, M, N, K, residual):
+    """Either side of the rule for the tile, in 128 x 128 tiles on 256 CUs: 232, 208, 240, 272 (twice), 357 and 416,
+    without a residual (64 x 64 tiles up to 224 or 256, and from 257 to 320) and with one (up to 384)."""
+    ops = _ops()
+    if not residual:
+        return test_split_linear_sizes(form, M, N, K, None)
+    g = torch.Generator(DEV).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=DEV)
+    kw, wd = _weight(ops, form, N, K, g)
+    buf = torch.randn(M, N, generator=g, device=DEV)
+    want = buf.double() + x.double() @ wd.t().contiguous()
+    ops.norm_linear(x, **kw, residual=buf, out=buf, compute_dtype=torch.float32)
+    assert ((buf - want).abs() <= _bound(x.double(), wd) + 2.0 ** -22 * want.abs() + 2.0 ** -22).all()
