@@ -39,12 +39,6 @@ namespace cortex {
 
 namespace {
 
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(n >= 0 && n < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((n & 15) | 0x70 | 0xF00 | ((n >> 4) << 14));
-}
-
 // pair d (values 2d, 2d + 1) of eight bf16 values, for the two-term dot products
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ bf16x2_t pair_of(const bf16x8& v, int d) {
@@ -54,25 +48,6 @@ __device__ __forceinline__ bf16x2_t pair_of(const bf16x8& v, int d) {
     case 2: return __builtin_shufflevector(v, v, 4, 5);
     default: return __builtin_shufflevector(v, v, 6, 7);
   }
-}
-
-// Direct-to-LDS transfer from a uniform base plus a 32-bit lane offset (global_load_lds in its
-// scalar-base form: one VGPR per transfer instead of a 64-bit address) into the LDS address m0
-// (wave-uniform: lane i writes m0 + SIZE * i), SIZE 16 (dwordx4) or 4 (dword).  The caller's
-// vmcnt waits order the reads.
-template <int SIZE>
-__device__ __forceinline__ void lds_dma_m0(const void* base, uint32_t voff, uint32_t m0) {
-  const uint64_t b = (uint64_t)(uintptr_t)base;
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
-  const uint64_t sb = ((uint64_t)hi << 32) | (uint64_t)lo;
-  const uint32_t m = __builtin_amdgcn_readfirstlane(m0);
-  if constexpr (SIZE == 16)
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sb), "s"(m)
-                 : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sb), "s"(m)
-                 : "memory", "m0");
 }
 
 // KS > 1 splits K over KS groups of WM x WN wavefronts, each streaming its own part of

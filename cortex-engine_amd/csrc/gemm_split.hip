@@ -37,23 +37,6 @@ namespace cortex {
 
 namespace {
 
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(n >= 0 && n < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((n & 15) | 0x70 | 0xF00 | ((n >> 4) << 14));
-}
-
-// 1 KiB per wavefront from a uniform address (lane i: 16 bytes at src + 16 i) into LDS address m0 +
-// 16 i; ordered by the caller's vmcnt waits.
-__device__ __forceinline__ void lds_dma_1k(const unsigned char* src, uint32_t lane16, uint32_t m0) {
-  const uint64_t b = (uint64_t)(uintptr_t)src;
-  const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) |
-                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
-  const uint32_t m = __builtin_amdgcn_readfirstlane(m0);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane16), "s"(sb), "s"(m)
-               : "memory");
-}
-
 constexpr int SP_BLK = 1024;  // bytes of one plane's 32 x 16 block
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -313,10 +296,10 @@ __global__ __launch_bounds__(256, TL::MINW) void gemm_split_kernel(SplitArgs g) 
   // transfer i of step kt into slot s
   auto issue_one = [&](int i, int kt, int s) __attribute__((always_inline)) {
     if (i < TL::AB)
-      lds_dma_1k(a_src[i] + (int64_t)kt * 6 * SP_BLK, lane16, lds0 + s * TL::STAGE + (wid * TL::AB + i) * SP_BLK);
+      lds_dma_m0<16>(a_src[i] + (int64_t)kt * 6 * SP_BLK, lane16, lds0 + s * TL::STAGE + (wid * TL::AB + i) * SP_BLK);
     else
-      lds_dma_1k(w_src[i - TL::AB] + (int64_t)kt * 2 * WP * SP_BLK, lane16,
-                 lds0 + s * TL::STAGE + TL::A_STAGE + (wid * TL::WB + i - TL::AB) * SP_BLK);
+      lds_dma_m0<16>(w_src[i - TL::AB] + (int64_t)kt * 2 * WP * SP_BLK, lane16,
+                     lds0 + s * TL::STAGE + TL::A_STAGE + (wid * TL::WB + i - TL::AB) * SP_BLK);
   };
   auto issue = [&](int kt, int s) __attribute__((always_inline)) {
 #pragma unroll

@@ -38,22 +38,6 @@ constexpr int GW_PATCH = 32 * GW_LD * 4;    // 8 KiB per wavefront, 16-byte chun
 constexpr int GW_LDS = GW_RING + 4 * GW_PATCH;
 static_assert(GW_LDS <= 160 * 1024, "LDS");
 
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(n >= 0 && n < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((n & 15) | 0x70 | 0xF00 | ((n >> 4) << 14));
-}
-
-// 1 KiB per wavefront, lane i: 16 bytes at base + voff into LDS address m0 + 16 i
-__device__ __forceinline__ void dma(const unsigned char* base, uint32_t voff, uint32_t m0) {
-  const uint64_t b = (uint64_t)(uintptr_t)base;
-  const uint64_t sb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32) |
-                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
-  const uint32_t m = __builtin_amdgcn_readfirstlane(m0);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sb), "s"(m)
-               : "memory");
-}
-
 struct WideArgs {
   int M, N, K;
   const unsigned char* x;
@@ -93,7 +77,7 @@ __global__ __launch_bounds__(256, 1) void gemm_wide_kernel(WideArgs g) {
   };
   auto issue = [&](int i, int kt, int s) __attribute__((always_inline)) {  // transfer i (0 .. 15) of stage kt
     const uint32_t to = lds0 + s * GW_STAGE + (i < 8 ? 0 : GW_OP) + (wid * 8 + (i & 7)) * 1024;
-    dma((i < 8 ? g.x : g.w) + kt * 128, i < 8 ? a_off[i & 7] : w_off[i & 7], to);
+    lds_dma_m0<16>((i < 8 ? g.x : g.w) + kt * 128, i < 8 ? a_off[i & 7] : w_off[i & 7], to);
   };
 
   // fragment addresses inside an operand's stage: row (lane % 32) of a 32-row tile, chunk 2 q + lane / 32
