@@ -133,9 +133,11 @@ def test_pack_plan_large_multi_chunk():
         np.testing.assert_array_equal(order.cpu().numpy(), p.order)
 
 
-@pytest.mark.parametrize("E,B", [(65536, 1024), (65537, 1024), (5000, 1025), (64, 1), (65536, 3)])
+@pytest.mark.parametrize("E,B", [(65536, 1024), (65537, 1024), (5000, 1025), (64, 1), (65536, 3), (4096, 1024), (4097, 1024),
+                                 (4096, 1025), (131072, 1024), (131073, 1024)])
 def test_pack_plan_path_boundaries(E, B):
-    """Either side of the one-launch plan's limits (B <= 1024, E <= 65536): same results."""
+    """Either side of the limits of the one-launch plan (B <= 1024, E <= 4096) and of the two-launch plan (B <=
+    1024, 2^17 counts: 128 chunks of 1024 events at 1024 samples): same results."""
     from cortex.kernels.pack import pack_plan
 
     rng = np.random.default_rng(E + B)
@@ -241,21 +243,22 @@ def _sorted_cases():
     b = np.sort(rng.integers(0, 21, 4000))
     b[2047], b[2048] = b[2048], b[2047] - 1 if b[2047] > 0 else 1
     cases["inversion_4000"] = (b, 21)
-    # above 4096 events the check runs wide (a workgroup per 256 events) before the plan kernel
+    # above 4096 events the check runs with the counts (a workgroup per 1024 events), whose sorted chunks write
+    # their part of the identity plan
     b = np.sort(rng.integers(0, 21, 20000))
     b[5119], b[5120] = b[5120], b[5119] - 1 if b[5119] > 0 else 1
     cases["inversion_wide"] = (b, 21)
     b = np.sort(rng.integers(0, 33, 20000))
-    b[256], b[255] = b[255], b[256] + 1  # an inversion across a 256-event range edge
+    b[256], b[255] = b[255], b[256] + 1  # an inversion inside the first chunk
     cases["inversion_wide_range_edge"] = (b, 34)
     b = np.sort(rng.integers(0, 30, 17000))
     b[16999] = 30
     cases["out_of_range_tail_wide"] = (b, 30)
     cases["sorted_4096"] = (np.sort(rng.integers(0, 33, 4096)), 33)
     cases["sorted_4097"] = (np.sort(rng.integers(0, 33, 4097)), 40)
-    cases["sorted_16447"] = (np.sort(rng.integers(0, 33, 16447)), 33)  # partial last wave of the wide check
-    # above 65536 events (or above 1024 samples) the general three-launch plan follows the wide
-    # check and returns at once when every range was sorted
+    cases["sorted_16447"] = (np.sort(rng.integers(0, 33, 16447)), 33)  # partial last chunk
+    # past 1024 samples (or 2^17 counts) the plan is three launches, of which the later two return at once when
+    # every chunk was sorted
     cases["sorted_70000"] = (np.sort(rng.integers(0, 200, 70000)), 200)
     b = np.sort(rng.integers(0, 200, 70000))
     b[60000], b[60001] = b[60001], b[60000] - 1 if b[60000] > 0 else 1
@@ -272,9 +275,8 @@ def _sorted_cases():
 
 @pytest.mark.parametrize("name", list(_sorted_cases()))
 def test_pack_plan_sorted_fast_path(name):
-    """Sorted batch indices take the identity plan (checked inside the plan kernel up to 4096
-    events, by the wide pack_sorted_kernel above, also ahead of the general three-launch plan
-    past 65536 events or 1024 samples); anything else found
+    """Sorted batch indices take the identity plan (checked inside the one-launch plan up to 4096
+    events, with the counts of each chunk above); anything else found
     there -- an inversion, an index out of range -- falls back to the full plan.  Same
     results as the oracle either way, with and without ranks; with the identity flag, a
     sorted in-range plan sets it (order is then the identity by definition) and any other
@@ -311,8 +313,8 @@ def test_pack_plan_sorted_fast_path(name):
                                               (16384, 32, False, False), (16384, 32, True, False),
                                               (70000, 2000, False, False), (70000, 2000, True, True)])
 def test_pack_plan_widen_rider(E, B, shuffle, rank):
-    """cortex_pack_plan_widen on every plan path (one launch up to 4096 events, the wide sorted
-    check, the three-launch plan with and without ranks, no events): the plan is exactly the
+    """cortex_pack_plan_widen on every plan path (one launch up to 4096 events, two launches, the
+    three-launch plan with and without ranks, no events): the plan is exactly the
     one without a rider, and the rider's int8 arrays (ragged sizes, one not a whole workgroup
     chunk) come out widened exactly."""
     from cortex.kernels import ops
