@@ -750,18 +750,20 @@ def linear_small(x: torch.Tensor, weight: torch.Tensor, weight_scale=None, bias=
     N = weight.shape[0]
     if weight.shape[1] != K:
         raise ValueError(f"inner dims differ: x has K={K}, weight has K={weight.shape[1]}")
-    if not x_frag:  # (expanded or overlapping rows are copied)
-        x = _row_major_2d(x)
+    ld_x, ld_res = x.stride(0), N
+    if not x_frag and (x.stride(1) != 1 or (M > 1 and ld_x < K)):  # (expanded or overlapping rows are copied)
+        x, ld_x = x.contiguous(), K
     if residual is not None:
         residual = _row_major_2d(residual)
+        if residual.shape[0] > 1:
+            ld_res = residual.stride(0)
     if out is None:
         out = torch.empty((ceil_div(M, 16) * 16 if out_frag else M, N), dtype=out_dtype, device=dev)
     g, b, eps = ln if ln is not None else (None, None, 0.0)
     nat.call("cortex_linear_small", M, N, K, nat.BF16_FRAG if x_frag else nat.code(x.dtype), nat.ptr(x),
-             x.stride(0) if x.shape[0] > 1 else K, nat.ptr(g), nat.ptr(b), float(eps),
+             ld_x if M > 1 else K, nat.ptr(g), nat.ptr(b), float(eps),
              nat.I8 if weight.dtype == torch.int8 else nat.BF16_FRAG, nat.ptr(weight), weight.stride(0),
-             nat.ptr(weight_scale), nat.ptr(bias), ACT[act], nat.ptr(residual),
-             residual.stride(0) if residual is not None and residual.shape[0] > 1 else N, int(res_rows),
+             nat.ptr(weight_scale), nat.ptr(bias), ACT[act], nat.ptr(residual), ld_res, int(res_rows),
              nat.BF16_FRAG if out_frag else nat.code(out.dtype), nat.ptr(out), out.stride(0) if M > 1 else N,
              nat.stream_of(dev))
     return out
