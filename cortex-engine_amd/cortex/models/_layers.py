@@ -21,6 +21,8 @@ bf16 compute (the default):
     image speed and no launch is added (``WeightWindow``).
     For a float nn.Linear the image is the weight rounded to bf16, as ``F.linear`` on
     bf16 inputs would use it.
+  * a linear of few rows reads its weight in MFMA fragment order (``frag_image``): used at few and at
+    many rows, it keeps both forms (2 bytes a parameter more).
 fp32 compute: int8 or fp32 weights, fp32 operands as exact sums of bf16 parts (gemm_split.hip), the
 norm applied where the rows are split.
 """

@@ -264,9 +264,10 @@ int cortex_bf16_gemm_form(int64_t M, int64_t N, int64_t K, int w_dtype, int out_
  * a: bf16 rows (gamma NULL; x_dtype 1, or 7 for rows in fragment order), or bf16(LayerNorm(x)) of fp32 rows
  * (x_dtype 0, gamma and beta given, fp32), its statistics computed by the call.  K 256, 512, 768 or 1024,
  * without LayerNorm also 2048 or 3072; w the (N, K) weight, w_dtype 7 for bf16 in fragment order
- * (cortex_frag_weight; ld_w ignored) or 3 for int8 rows (8-byte aligned, the same results), N a multiple of 16; rows 16-byte aligned; w_scale, bias, residual optional fp32; act 0 or 1 (erf-GELU); out
- * fp32 (0, may be residual), bf16 (1) or bf16 in fragment order (7: as cortex_frag_weight's, M rounded up
- * to 16 rows, N a multiple of 32; the row strides are ignored); res_rows 0 means M. */
+ * (cortex_frag_weight; ld_w ignored) or 3 for int8 rows (8-byte aligned, the same results), N a multiple
+ * of 16; rows 16-byte aligned; w_scale, bias, residual optional fp32; act 0 or 1 (erf-GELU); out fp32 (0,
+ * may be residual), bf16 (1) or bf16 in fragment order (7: as cortex_frag_weight's, M rounded up to 16
+ * rows, N a multiple of 32; the row strides are ignored); res_rows 0 means M. */
 int cortex_linear_small(int64_t M, int64_t N, int64_t K, int x_dtype, const void* x, int64_t ld_x,
                         const float* gamma, const float* beta, float eps, int w_dtype, const void* w, int64_t ld_w,
                         const float* w_scale, const float* bias, int act, const float* residual, int64_t ld_res,
@@ -274,8 +275,8 @@ int cortex_linear_small(int64_t M, int64_t N, int64_t K, int x_dtype, const void
 
 /* The fp32-compute form of cortex_norm_linear on the bf16 matrix cores (the fp32 rows of
  * cortex/kernels/fused_rmsnorm.py:239-301 and of QuantizedLinear, calibrate.py:225-228): every
- * fp32 operand as the exact sum of three bf16 parts, products and sums in fp32 (an int8 weight is
- * one part).  x, residual and out fp32; w int8 (N, K) or fp32 in (N, K) (w_layout 0) or (K, N) (1);
+ * fp32 operand as the exact sum of three bf16 parts (a value below 2^-110 off by up to 2^-134), products and
+ * sums in fp32 (an int8 weight is one part).  x, residual and out fp32; w int8 (N, K) or fp32 in (N, K) (w_layout 0) or (K, N) (1);
  * norm 0 none, 1 LayerNorm, 2 RMS, its statistics computed by the call (gamma and beta in
  * gamma_dtype 0, 1 or 2); w_scale, bias optional fp32; act, residual and res_rows as
  * cortex_norm_linear; out may be residual.  The workspace (16-byte aligned) holds the parts of the
