@@ -757,8 +757,13 @@ def linear_small(x: torch.Tensor, weight: torch.Tensor, weight_scale=None, bias=
         residual = _row_major_2d(residual)
         if residual.shape[0] > 1:
             ld_res = residual.stride(0)
+    m_out = ceil_div(M, 16) * 16 if out_frag else M
     if out is None:
-        out = torch.empty((ceil_div(M, 16) * 16 if out_frag else M, N), dtype=out_dtype, device=dev)
+        out = torch.empty((m_out, N), dtype=out_dtype, device=dev)
+    elif out.shape[0] < m_out:
+        raise ValueError(f"out must hold {m_out} rows of {N} values, got shape {tuple(out.shape)}")
+    if x_frag and x.shape[0] < ceil_div(M, 16) * 16:
+        raise ValueError(f"{M} rows in fragment order need {ceil_div(M, 16) * 16}, got {x.shape[0]}")
     g, b, eps = ln if ln is not None else (None, None, 0.0)
     nat.call("cortex_linear_small", M, N, K, nat.BF16_FRAG if x_frag else nat.code(x.dtype), nat.ptr(x),
              ld_x if M > 1 else K, nat.ptr(g), nat.ptr(b), float(eps),

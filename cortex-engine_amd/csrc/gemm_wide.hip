@@ -15,7 +15,7 @@
 // at a time through LDS of its own, so that residual and output rows move in whole 256-byte pieces and a lane's
 // scale and bias columns stay the same.
 //
-// Against 256 x 128 tiles of eight wavefronts (repeated alone, over several boxes): 32768 x 512 x 2048 87.6 -> 76 .. 79 us,
+// Against 256 x 128 tiles of eight wavefronts (repeated alone, on several GPUs): 32768 x 512 x 2048 87.6 -> 76 .. 79 us,
 // 65536 x 512 x 2048 178.7 -> 160 .. 170, 36864 x 768 x 3072 225 -> 194 .. 198.  (With a bf16 output and the GELU in place of the residual, K = 512, it is the
 // slower form, 205 against 216 us at 65536 x 2048 x 512: one wavefront per SIMD has nothing to overlap the
 // epilogue's arithmetic with.)

@@ -181,3 +181,19 @@ def test_output_buffer_with_more_rows(M):
                 ops.norm_linear(x, weight=w, out_dtype=dtype, out=out[:0])
             with pytest.raises((ValueError, RuntimeError)):
                 ops.norm_linear(x, weight=lin.weight, out_dtype=dtype, out=out[:M - 1])
+
+
+def test_buffers_too_small_are_refused():
+    """Outputs, and rows in fragment order, of fewer rows than a launch writes or reads."""
+    from cortex.kernels import ops
+
+    _, x, w, s, _ = _case(20, 64, 256, 0)
+    xb, wf = x.bfloat16(), ops.frag_weight(w)
+    xf = ops.frag_weight(torch.zeros(32, 256, dtype=torch.bfloat16, device=DEV))
+    with pytest.raises(ValueError):
+        ops.linear_small(xb, wf, s, out=torch.empty(19, 64, device=DEV))
+    with pytest.raises(ValueError):
+        ops.linear_small(xb, wf, s, out=torch.empty(20, 64, dtype=torch.bfloat16, device=DEV), out_frag=True)
+    with pytest.raises(ValueError):
+        ops.linear_small(xf[:16], wf, s, rows=20)
+    assert ops.linear_small(xf, wf, s, rows=20).shape == (20, 64)
